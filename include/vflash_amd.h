@@ -342,6 +342,27 @@ int vflash_fp8_linear_lora_branches(const void* a, const float* sa, int64_t lda,
                                     float strength, void* out, int64_t ldo, int64_t plane_cols,
                                     int64_t plane_stride, void* stream);
 
+/* Weight-only linear: out[m, n] = bf16(sum_k x[m, k] * w[n, k] + bias[n]) with the weight
+ * restored inside the GEMM, w = bf16(e4m3(code) * sw[n]).
+ * Replaces (weight.float() * scale).to(bfloat16) followed by F.linear in the weight-only mode of
+ *   RowFP8Execution.linear (src/vflash/native/h3_fp8_linear.py:75-108).
+ *   x    bf16 [m, k] (ldx elements, a multiple of 8); w: E4M3 codes [n, k] (ldw bytes, a
+ *        multiple of 16); sw: fp32 [n]; bias: bf16 [n] or NULL; out: bf16 [m, n] (ldo elements,
+ *        a multiple of 8); all 16-byte aligned
+ *   k a multiple of 16, n a multiple of 8
+ */
+int vflash_w8a16_linear(const void* x, int64_t ldx, const void* w, const float* sw, int64_t ldw,
+                        int64_t m, int64_t n, int64_t k, const void* bias, void* out, int64_t ldo,
+                        void* stream);
+
+/* The weight of the weight-only mode, restored: out[n, k] = bf16(e4m3(code) * sw[n]), the value of
+ * (weight.float() * scale).to(bfloat16) (src/vflash/native/h3_fp8_linear.py:75-108).
+ *   w: E4M3 codes [n, k] (ldw bytes, a multiple of 16; 16-byte aligned); sw: fp32 [n];
+ *   out: bf16 [n, k], contiguous, 16-byte aligned; k a multiple of 16
+ */
+int vflash_restore_rows_bf16(const void* w, const float* sw, int64_t ldw, int64_t n, int64_t k,
+                             void* out, void* stream);
+
 /*
  * NVFP4-weight linear (W4A8: E4M3 per-token activations, E2M1 weights with
  * E4M3 scales per 16-element K block and an fp32 output multiplier).  A more

@@ -82,6 +82,11 @@ SIGNATURES: dict[str, tuple[list, object]] = {
         _I32,
     ),
     "vflash_fp8_gemm_tiling": ([_I64, _I64, _I64, _I64], _I32),
+    "vflash_w8a16_linear": (
+        [_P, _I64, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _P],
+        _I32,
+    ),
+    "vflash_restore_rows_bf16": ([_P, _P, _I64, _I64, _I64, _P, _P], _I32),
     "vflash_nvfp4_linear": (
         [_P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _P, _P, _I64, _P],
         _I32,

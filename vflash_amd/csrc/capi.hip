@@ -29,6 +29,9 @@ hipError_t launch_nvfp4_quant(const uint16_t*, bool, int64_t, int64_t, int64_t, 
 hipError_t launch_nvfp4_w4a4(const uint8_t*, int64_t, const uint8_t*, const uint8_t*,
                              const uint8_t*, const float*, int64_t, int64_t, int64_t,
                              const uint16_t*, uint16_t*, int64_t, int, hipStream_t);
+hipError_t launch_w8a16(const GemmParams&, hipStream_t);
+hipError_t launch_restore_rows(const uint8_t*, const float*, int64_t, int64_t, int64_t, uint16_t*,
+                               hipStream_t);
 hipError_t launch_nvfp4(const uint8_t*, const float*, int64_t, const uint8_t*, const uint8_t*,
                         const float*, int64_t, int64_t, int64_t, const uint16_t*, uint16_t*, int64_t,
                         int, hipStream_t);
@@ -379,6 +382,29 @@ int vflash_fp8_linear_lora_branches(const void* a, const float* sa, int64_t lda,
   p.lora_t_branch = branches > 1 ? t_branch : 0;
   for (int b = 0; b < branches; ++b) p.lora_scale[b] = scales[b];
   return status(vfa::launch_fp8_gemm(p, vfa::EPI_LORA, static_cast<hipStream_t>(stream)));
+}
+
+int vflash_w8a16_linear(const void* x, int64_t ldx, const void* w, const float* sw, int64_t ldw,
+                        int64_t m, int64_t n, int64_t k, const void* bias, void* out, int64_t ldo,
+                        void* stream) {
+  if (!x || !w || !sw || !out || m < 1 || n < 8 || n % 8 || k < 16 || k % 16) return VFLASH_EINVAL;
+  if (ldx < k || ldx % 8 || ldw < k || ldw % 16 || ldo < n || ldo % 8) return VFLASH_EINVAL;
+  if (!aligned(x, 16) || !aligned(w, 16) || !aligned(sw, 16) || !aligned(out, 16) ||
+      (bias && !aligned(bias, 16)))
+    return VFLASH_EINVAL;
+  if (512 * ldx >= (int64_t(1) << 31) || 256 * ldw >= (int64_t(1) << 31)) return VFLASH_EINVAL;
+  vfa::GemmParams p = base_params(x, nullptr, 2 * ldx, w, sw, ldw, m, n, k, bias, out, ldo);
+  return status(vfa::launch_w8a16(p, static_cast<hipStream_t>(stream)));
+}
+
+int vflash_restore_rows_bf16(const void* w, const float* sw, int64_t ldw, int64_t n, int64_t k,
+                             void* out, void* stream) {
+  if (!w || !sw || !out || n < 1 || n >= (int64_t(1) << 31) || k < 16 || k % 16 || ldw < k || ldw % 16)
+    return VFLASH_EINVAL;
+  if (k >= (int64_t(1) << 31) || !aligned(w, 16) || !aligned(sw, 4) || !aligned(out, 16))
+    return VFLASH_EINVAL;
+  return status(vfa::launch_restore_rows(static_cast<const uint8_t*>(w), sw, n, k, ldw,
+                                         static_cast<uint16_t*>(out), static_cast<hipStream_t>(stream)));
 }
 
 int vflash_nvfp4_linear(const void* a, const float* sa, int64_t lda, const void* w_packed,

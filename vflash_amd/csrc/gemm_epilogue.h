@@ -448,9 +448,16 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p,
           // v_cvt_pk_bf16_f32 for the pair.
           static_for<2>([&](auto h) {
             constexpr int i0 = 2 * h, i1 = 2 * h + 1;
-            float y0 = acc[nb][mb][g * 4 + i0] * sam[mb] * sv[g][i0];
-            float y1 = acc[nb][mb][g * 4 + i1] * sam[mb] * sv[g][i1];
-            if constexpr (has_bias) {
+            float y0 = acc[nb][mb][g * 4 + i0];
+            float y1 = acc[nb][mb][g * 4 + i1];
+            if constexpr (EPI == EPI_LINEAR) {
+              y0 += bv[g][i0];
+              y1 += bv[g][i1];
+            } else {
+              y0 = y0 * sam[mb] * sv[g][i0];
+              y1 = y1 * sam[mb] * sv[g][i1];
+            }
+            if constexpr (has_bias && EPI != EPI_LINEAR) {
               y0 = round_bf16_wide(y0) + bv[g][i0];
               y1 = round_bf16_wide(y1) + bv[g][i1];
             }

@@ -9,6 +9,7 @@ namespace vfa {
 // gate-residual (phase 2) and the SwiGLU activation (phase 2).
 enum {
   EPI_BIAS = 0,
+  EPI_LINEAR = 1,  // bf16(acc + bias): no scales, one rounding (weight-only GEMM)
   EPI_GATE = 2,
   EPI_LORA = 3,
   EPI_SWIGLU = 4,

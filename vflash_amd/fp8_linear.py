@@ -120,6 +120,9 @@ class RowFP8Execution:
             if isinstance(value, QuantizedRows):
                 raise ValueError("pre-quantized activations require the w8a8 mode")
             self.calls["weight_only"] += 1
+            output = kernels.weight_only_linear(value, weight, scale, bias)
+            if output is not None:
+                return output
             restored = (weight.float() * scale).to(value.dtype)
             return torch.nn.functional.linear(value, restored, bias)
         if not w8a8_supported(value):

@@ -479,6 +479,67 @@ GEMM_TILINGS = ("256x256", "256x192", "256x128", "128x192", "128x128", "128x128 
                 "128x64", "64x64")
 
 
+def _plain(*tensors) -> bool:
+    """Strided tensors that no tracer, subclass, transform or pending sign is attached to."""
+    return all(
+        t is None
+        or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided and not t.is_neg())
+        for t in tensors
+    )
+
+
+def _eager_inference(*tensors) -> bool:
+    """True where a call is plain eager arithmetic that nothing records: no gradient
+    or forward-mode tangent to carry, no autocast, mode, tracer or transform active."""
+    return not (
+        (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))
+        or torch.is_autocast_enabled("cuda")
+        or torch.jit.is_tracing()
+        or torch.compiler.is_compiling()
+        or torch._C._len_torch_dispatch_stack()
+        or torch._C._len_torch_function_stack()
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch.autograd.forward_ad._current_level >= 0
+    ) and _plain(*tensors)
+
+
+# Rows up to which the GEMM that restores the weight in registers is ahead of one
+# pass that writes it as BF16 followed by a plain BF16 GEMM.
+WEIGHT_ONLY_FUSED_ROWS = 1024
+
+
+def weight_only_linear(value, weight, scale, bias=None):
+    """``F.linear(value, (weight.float() * scale).to(bfloat16), bias)`` as one GEMM that
+    restores the weight on the fly, or None where a call is outside the kernel's forms
+    (and the caller takes the torch expression): BF16 rows on the current gfx950 device,
+    K % 16 == 0, N % 8 == 0, 16-byte aligned operands with unit column stride, and
+    nothing that records the call (``_eager_inference``)."""
+    device = value.device
+    if (value.dtype != torch.bfloat16 or not _lib.is_gfx950(device)
+            or not _eager_inference(value, weight, scale, bias)
+            or device.index != torch.cuda.current_device()):
+        return None
+    n, k = weight.shape
+    matrix = value.reshape(-1, k)
+    rows = matrix.shape[0]
+    ldx, ldw = matrix.stride(0) if rows > 1 else k, weight.stride(0) if n > 1 else k
+    if (k % 16 or n % 8 or rows < 1 or matrix.stride(1) != 1 or ldx < k or ldx % 8 or ldx >= 1 << 22
+            or weight.stride(1) != 1 or ldw < k or ldw % 16 or ldw >= 1 << 23
+            or not scale.is_contiguous() or (bias is not None and not bias.is_contiguous())):
+        return None
+    x_ptr, w_ptr, s_ptr, b_ptr = ptr(matrix), ptr(weight), ptr(scale), ptr(bias)
+    if (x_ptr | w_ptr | s_ptr | (b_ptr or 0)) % 16:
+        return None
+    if rows > WEIGHT_ONLY_FUSED_ROWS:
+        restored = torch.empty((n, k), device=device, dtype=torch.bfloat16)
+        call("vflash_restore_rows_bf16", w_ptr, s_ptr, ldw, n, k, ptr(restored), stream_of(device))
+        return torch.nn.functional.linear(value, restored, bias)
+    out = torch.empty((*value.shape[:-1], n), device=device, dtype=torch.bfloat16)
+    call("vflash_w8a16_linear", x_ptr, ldx, w_ptr, s_ptr, ldw, rows, n, k, b_ptr, ptr(out), n,
+         stream_of(device))
+    return out
+
+
 def nvfp4_gemm(codes, act_scale, packed, block_scales, alpha, rows, bias=None):
     """W4A8 NVFP4-weight GEMM: out[rows, N] bf16."""
     if codes.dtype != E4M3 or codes.ndim != 2 or codes.stride(1) != 1:
