@@ -31,8 +31,10 @@ __device__ __forceinline__ float half_hi(uint32_t w) {
   return bf16_hi(w);
 }
 
-// One wave per row, four rows per workgroup.  Lane l of pass t reads the 8
-// elements 512 t + 8 l .. +7 (16 bytes; the wave reads 1 KB contiguously), so
+// One wave per row segment, four rows per workgroup; gridDim.y splits each row
+// into runs of whole 64-element groups (blocks are independent, and few rows
+// would leave the GPU idle otherwise).  Lane l of pass t reads the 8 elements
+// 512 t + 8 l .. +7 of the segment (16 bytes; four passes' loads are in flight; the wave reads 1 KB contiguously), so
 // a 16-element block is a lane pair: the block maximum takes one shuffle, and
 // each lane writes its 4 packed bytes.  The four scales of a 128x4 word (four
 // consecutive blocks) come from lanes 8u, 8u + 2, 8u + 4, 8u + 6 and are
@@ -49,8 +51,10 @@ __global__ void __launch_bounds__(256) nvfp4_quant_rows(const uint16_t* __restri
   if (row >= m_pad) return;
   const int64_t groups = k / 64;  // 128x4 scale words per row
   uint8_t* srow = scales + (row / 128) * groups * 512 + (row % 32) * 16 + ((row % 128) / 32) * 4;
+  const int g0 = (int)(groups * blockIdx.y / gridDim.y);
+  const int g1 = (int)(groups * (blockIdx.y + 1) / gridDim.y);
   if (row >= m) {
-    for (int64_t gi = lane; gi < groups; gi += 64) *reinterpret_cast<uint32_t*>(srow + gi * 512) = 0u;
+    for (int64_t gi = g0 + lane; gi < g1; gi += 64) *reinterpret_cast<uint32_t*>(srow + gi * 512) = 0u;
     return;
   }
   const float gsf = *global_sf;
@@ -58,45 +62,57 @@ __global__ void __launch_bounds__(256) nvfp4_quant_rows(const uint16_t* __restri
   constexpr float SIXTH = 1.0f / 6.0f;
   const v4i* xr = reinterpret_cast<const v4i*>(x + row * ldx);
   uint32_t* cr = reinterpret_cast<uint32_t*>(codes + row * ldc);
-  const int nvec = (int)(k / 8);
-  for (int base = 0; base < nvec; base += 64) {  // uniform over the wave: shuffles below
-    const int j = base + lane;
-    const bool live = j < nvec;  // k % 64 == 0: whole 8-lane groups are live together
-    const v4i v = live ? __builtin_nontemporal_load(xr + j) : v4i{};
-    float amax = 0.0f;
+  const int nvec = 8 * g1;
+  for (int base0 = 8 * g0; base0 < nvec; base0 += 256) {  // uniform over the wave: shuffles below
+    v4i in[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t w = (uint32_t)v[e];
-      amax = fmaxf(amax, fmaxf(fabsf(half_lo<F16>(w)), fabsf(half_hi<F16>(w))));
+    for (int t = 0; t < 4; ++t) {
+      const int j = base0 + 64 * t + lane;
+      in[t] = j < nvec ? __builtin_nontemporal_load(xr + j) : v4i{};
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 1, 64));  // the block: this lane and its pair
-    const float sff = fminf(gsf * (amax * SIXTH), 448.0f);
-    const uint32_t sfc = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(sff, sff, 0, false) & 0xffu;
-    const float sf = e4m3_to_f32(sfc);
-    const float scale = sf != 0.0f ? 1.0f / (sf * inv_gsf) : 0.0f;
-    uint32_t word = 0u;
-    static_for<4>([&](auto e) {
-      const uint32_t w = (uint32_t)v[(int)e];
-      const float lo = fminf(fmaxf(half_lo<F16>(w) * scale, -6.0f), 6.0f);
-      const float hi = fminf(fmaxf(half_hi<F16>(w) * scale, -6.0f), 6.0f);
-      word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, lo, hi, 1.0f, (int)e);
-    });
-    const uint32_t s2 = (uint32_t)__shfl_down((int)sfc, 2, 64);
-    const uint32_t s4 = (uint32_t)__shfl_down((int)sfc, 4, 64);
-    const uint32_t s6 = (uint32_t)__shfl_down((int)sfc, 6, 64);
-    if (live) {
-      cr[j] = word;
-      if ((lane & 7) == 0)
-        *reinterpret_cast<uint32_t*>(srow + (int64_t)(j / 8) * 512) =
-            sfc | (s2 << 8) | (s4 << 16) | (s6 << 24);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (base0 + 64 * t >= nvec) break;
+      const int j = base0 + 64 * t + lane;
+      const bool live = j < nvec;  // whole 8-lane groups are live together
+      const v4i v = in[t];
+      float amax = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w = (uint32_t)v[e];
+        amax = fmaxf(amax, fmaxf(fabsf(half_lo<F16>(w)), fabsf(half_hi<F16>(w))));
+      }
+      amax = fmaxf(amax, __shfl_xor(amax, 1, 64));  // the block: this lane and its pair
+      const float sff = fminf(gsf * (amax * SIXTH), 448.0f);
+      const uint32_t sfc = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(sff, sff, 0, false) & 0xffu;
+      const float sf = e4m3_to_f32(sfc);
+      const float scale = sf != 0.0f ? 1.0f / (sf * inv_gsf) : 0.0f;
+      uint32_t word = 0u;
+      static_for<4>([&](auto e) {
+        const uint32_t w = (uint32_t)v[(int)e];
+        const float lo = fminf(fmaxf(half_lo<F16>(w) * scale, -6.0f), 6.0f);
+        const float hi = fminf(fmaxf(half_hi<F16>(w) * scale, -6.0f), 6.0f);
+        word = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, lo, hi, 1.0f, (int)e);
+      });
+      const uint32_t s2 = (uint32_t)__shfl_down((int)sfc, 2, 64);
+      const uint32_t s4 = (uint32_t)__shfl_down((int)sfc, 4, 64);
+      const uint32_t s6 = (uint32_t)__shfl_down((int)sfc, 6, 64);
+      if (live) {
+        cr[j] = word;
+        if ((lane & 7) == 0)
+          *reinterpret_cast<uint32_t*>(srow + (int64_t)(j / 8) * 512) =
+              sfc | (s2 << 8) | (s4 << 16) | (s6 << 24);
+      }
     }
   }
 }
 
+unsigned row_segments(int64_t rows, int64_t k);
+
 hipError_t launch_nvfp4_quant(const uint16_t* x, bool f16, int64_t m, int64_t k, int64_t ldx,
                               const float* global_sf, uint8_t* codes, int64_t ldc,
                               uint8_t* scales, int64_t m_pad, hipStream_t s) {
-  const dim3 grid((unsigned)((m_pad + 3) / 4));
+  const dim3 grid((unsigned)((m_pad + 3) / 4), row_segments(m_pad, k));
   if (f16)
     nvfp4_quant_rows<true><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad);
   else

@@ -126,21 +126,21 @@ __device__ __forceinline__ uint2 quant8(v4i v, const RowDivisor& d) {
 }
 
 // Codes of one row held in registers: vector i of this lane is element
-// vector lane + 64 i of the row (i < VPL, lane + 64 i < nvec).
-template <int VPL>
+// vector lane + STEP i of the row (i < VPL, lane + STEP i < nvec).
+template <int VPL, int STEP = 64>
 __device__ __forceinline__ void quant_row_regs(uint2* cr, const v4i (&v)[VPL], int lane, int nvec,
                                                float scale, float amax) {
   const RowDivisor d = row_divisor(scale, amax);
   if (d.fast) {
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int j = lane + 64 * i;
+      const int j = lane + STEP * i;
       if (j < nvec) cr[j] = quant8<true>(v[i], d);
     }
   } else {
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int j = lane + 64 * i;
+      const int j = lane + STEP * i;
       if (j < nvec) cr[j] = quant8<false>(v[i], d);
     }
   }
