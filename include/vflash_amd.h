@@ -154,7 +154,9 @@ int64_t vflash_swiglu_parts(int64_t n);
  * m x n output on a device with `compute_units` CUs (a host-side query; no
  * device work).  0: 256x256, 1: 256x192, 2: 256x128, 3: 128x192, 4: 128x128
  * (two workgroups per CU), 5: 128x128 (one per CU, grids of one round),
- * 6: 128x64, 7: 64x64.  The SwiGLU entries always use 256x256.  No tiling
+ * 6: 128x64, 7: 64x64.  The SwiGLU entries always use 256x256.  The plain and
+ * gate-residual entries may run 256x256 tiles with a last round of smaller ones
+ * where this answers 256x256 or 256x192.  No tiling
  * changes a result bit; this exists so that tests can aim shapes at each one.
  * branch_cols > 0 (a multiple of 32): the choice of a LoRA entry with adapter
  * branches that wide, which takes only tilings whose wave width (half the tile

@@ -24,10 +24,12 @@
 // The LoRA delta may come from up to three adapter branches with their own
 // scales, each owning a contiguous run of output columns (the Q/K/V adapters of
 // a merged projection, h3_native_denoiser.py:301-316, h3_fused_ops.py:900-980).
-#include "fp8_gemm_pipe.h"
+#include "fp8_gemm_mixed.h"
 
 namespace vfa {
 
+extern template hipError_t launch_mixed<EPI_BIAS>(const GemmParams&, int64_t, int, hipStream_t);
+extern template hipError_t launch_mixed<EPI_GATE>(const GemmParams&, int64_t, int, hipStream_t);
 extern template hipError_t launch_tiling<EPI_BIAS>(const GemmParams&, int, hipStream_t);
 extern template hipError_t launch_tiling<EPI_GATE>(const GemmParams&, int, hipStream_t);
 extern template hipError_t launch_tiling<EPI_LORA>(const GemmParams&, int, hipStream_t);
@@ -111,6 +113,24 @@ int tiling_group_m(int tiling, int64_t tile_cols) {
   return tile_cols <= 48 ? 4 : 3;
 }
 
+// Whether the last round of a 256x256 grid is split into smaller tiles, so that
+// its few tiles spread over all CUs (bit-identical: every tiling is).  With two
+// or more whole rounds and at most half a round left, as 256x128 (one round of
+// them), in microseconds: 4095 x 5120 x 13824 235 -> 225 (3.375 rounds), 8190 x
+// 5376 x 7168 251 -> 234 (3.5), 20000 x 3072 x 5120 271 -> 261 (6.17), gate-residual
+// 32760 x 14336 x 5376 1941 -> 1913 (10.5).  With one whole round, where the
+// 256x192 tiling's 1.5 rounds beat two, with at most a quarter round left, as
+// 128x128: 4095 x 5120 x 5120 93 -> 88.5 (1.25 rounds), with gate-residual 123 ->
+// 111 and at K = 13824 259 -> 241.  More left than that is slower: 4200 x 5376 x
+// 5376 102 -> 115 (1.40 rounds), 12000 x 5120 x 13824 606 -> 618 (9.91), 5000 x 5120
+// x 5120 112 -> 124 (1.56).
+static int mixed_tail(const GemmParams& p, int tiling, int64_t tiles, int64_t cus) {
+  const int64_t full = tiles / cus, rem = tiles % cus;
+  if (p.k % 128 || rem == 0 || full < 1) return MIXED_NONE;
+  if (full >= 2) return tiling == GEMM_256x256 && 2 * rem <= cus ? MIXED_256x128 : MIXED_NONE;
+  return tiling == GEMM_256x192 && 4 * rem <= cus ? MIXED_128x128 : MIXED_NONE;
+}
+
 // GemmParams::group_m is set here from the tiling.
 hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
   GemmParams p = params;
@@ -124,6 +144,15 @@ hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
       pick_tiling(p.m, p.n, compute_units(), epi_lora(epi) ? p.lora_branch_cols : 0);
   if (tiling < 0) return hipErrorInvalidValue;
   p.group_m = tiling_group_m(tiling, (p.n + kTilings[tiling].bn - 1) / kTilings[tiling].bn);
+  if (epi == EPI_BIAS || epi == EPI_GATE) {
+    const int64_t tiles = ((p.m + 255) / 256) * ((p.n + 255) / 256), cus = compute_units();
+    const int tail = mixed_tail(p, tiling, tiles, cus);
+    if (tail != MIXED_NONE) {
+      p.group_m = tiling_group_m(GEMM_256x256, (p.n + 255) / 256);
+      return epi == EPI_BIAS ? launch_mixed<EPI_BIAS>(p, tiles / cus * cus, tail, s)
+                             : launch_mixed<EPI_GATE>(p, tiles / cus * cus, tail, s);
+    }
+  }
   switch (epi) {
     case EPI_BIAS: return launch_tiling<EPI_BIAS>(p, tiling, s);
     case EPI_GATE: return launch_tiling<EPI_GATE>(p, tiling, s);

@@ -9,9 +9,15 @@
 
 namespace vfa {
 
-// Logical tile index for this workgroup.  Workgroup b is dispatched to XCD
-// b % 8; renumbering gives each XCD a contiguous run of logical tiles, and a
-// grouped (GROUP_M tall) column sweep keeps the tiles that are resident on one
+// Logical tile index for workgroup b of nwg.  Workgroup b is dispatched to XCD
+// b % 8; renumbering gives each XCD a contiguous run of logical tiles.
+__device__ __forceinline__ int xcd_order(int b, int nwg) {
+  const int q = nwg >> 3, r = nwg & 7;
+  const int x = b & 7, i = b >> 3;
+  return x * q + min(x, r) + i;
+}
+
+// A grouped (GROUP_M tall) column sweep keeps the tiles that are resident on one
 // XCD at the same time sharing A rows and W rows in that XCD's L2.
 __device__ __forceinline__ void grouped_tile(int logical, int tiles_m, int tiles_n, int group_m,
                                              int& tm, int& tn) {
@@ -26,11 +32,7 @@ __device__ __forceinline__ void grouped_tile(int logical, int tiles_m, int tiles
 
 __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int group_m, int& tm,
                                             int& tn) {
-  const int nwg = gridDim.x;
-  const int b = blockIdx.x;
-  const int q = nwg >> 3, r = nwg & 7;
-  const int x = b & 7, i = b >> 3;
-  grouped_tile(x * q + min(x, r) + i, tiles_m, tiles_n, group_m, tm, tn);
+  grouped_tile(xcd_order((int)blockIdx.x, (int)gridDim.x), tiles_m, tiles_n, group_m, tm, tn);
 }
 
 // Adapter operands of the LoRA epilogues.  A rank step covers 16 rank
