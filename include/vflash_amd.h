@@ -159,8 +159,8 @@ int64_t vflash_swiglu_parts(int64_t n);
  * where this answers 256x256 or 256x192.  No tiling
  * changes a result bit; this exists so that tests can aim shapes at each one.
  * branch_cols > 0 (a multiple of 32): the choice of a LoRA entry with adapter
- * branches that wide, which takes only tilings whose wave width (half the tile
- * width) divides branch_cols.
+ * branches that wide: the best of the tilings whose wave width (half the tile width)
+ * divides branch_cols (a launch may still run 256x192, whose epilogue splits a wave).
  */
 int vflash_fp8_gemm_tiling(int64_t m, int64_t n, int64_t compute_units, int64_t branch_cols);
 

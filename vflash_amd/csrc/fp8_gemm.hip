@@ -140,9 +140,21 @@ hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
     if (epi == EPI_SWIGLU_LORA) return launch_pipe<EPI_SWIGLU_LORA, PipeCfg<256, 256, SPLIT_RING, 0>>(p, s);
     return launch_pipe<EPI_SWIGLU, PipeCfg<256, 256, SPLIT_RING, 0>>(p, s);
   }
-  const int tiling =
+  int tiling =
       pick_tiling(p.m, p.n, compute_units(), epi_lora(epi) ? p.lora_branch_cols : 0);
   if (tiling < 0) return hipErrorInvalidValue;
+  // Adapter branches that 256x192 tiles would cut inside a wave: the query's
+  // choice leaves that tiling out, but its epilogue takes each 32-column block's
+  // branch by itself, so the launch may use it where it is the best one.  Merged
+  // QKV of 1024 rows at K 5376, 3 x 7168 columns, rank 128: 139 us as 256x128, 126
+  // as 256x192 (148 with the adapter gathered block by block in the epilogue);
+  // rank 16 121 and 112.
+  if (epi_lora(epi) && p.lora_branch_cols % 32 == 0 &&
+      pick_tiling(p.m, p.n, compute_units(), 0) == GEMM_256x192)
+    tiling = GEMM_256x192;
+  // That tile stages adapter rows through 32-bit buffer offsets.
+  if (epi_lora(epi) && tiling == GEMM_256x192 && (p.ldt >= (1 << 21) || p.ldb >= (1 << 21)))
+    tiling = p.lora_branch_cols % 64 ? GEMM_128x64 : GEMM_256x128;
   p.group_m = tiling_group_m(tiling, (p.n + kTilings[tiling].bn - 1) / kTilings[tiling].bn);
   if (epi == EPI_BIAS || epi == EPI_GATE) {
     const int64_t tiles = ((p.m + 255) / 256) * ((p.n + 255) / 256), cus = compute_units();

@@ -81,9 +81,8 @@ __device__ __forceinline__ int block_col(int wn, int nb) {
   return wave_col<BN, WN, SWIGLU>(wn) + block_off<BN, WN, SWIGLU>(nb);
 }
 
-// The adapter branch of a wave's columns, from its first column `col`: the
-// offset of its t columns and its scale.  A wave's columns lie in one branch
-// (the launcher picks a tiling whose wave width divides lora_branch_cols).
+// The adapter branch of a 32-column block, from its first column `col`: the
+// offset of its t columns and its scale.  Branches are whole blocks wide.
 struct LoraBranch {
   int64_t toff;
   float scale;
@@ -110,6 +109,7 @@ __device__ __forceinline__ void lora_blocks(const GemmParams& p, int64_t m0, int
   constexpr int WM = BM / WGM, WN = BN / WGN, MB = WM / 32, NB = WN / 32;
   constexpr int RS = 8;  // rank steps of 16: rank <= 128
   const int fr = lane & 31, fh = lane >> 5;
+  // The tiles that use it only take branches of whole waves.
   const LoraBranch br = lora_branch(p, tile_column<BN, SWIGLU>(p, n0, block_col<BN, WN, SWIGLU>(wn, 0)));
   v8s bf[NB][RS], tf[MB][RS];
   static_for<NB>([&](auto nb) {
@@ -136,6 +136,84 @@ __device__ __forceinline__ void lora_blocks(const GemmParams& p, int64_t m0, int
       d[nb * MB + mb] = acc;
     });
   });
+}
+
+// LoRA products of one wave's blocks after the main loop, d[nb * MB + mb], with
+// the operands staged in LDS: the rows of t and of B are DMA'd once per tile
+// (256-byte rows, whole lines) instead of being gathered 16 bytes a lane, block
+// by block, from global memory.  Row r of either operand holds rank chunk c (8
+// positions) in slot c ^ (r % 16); chunks at or past the rank read as zeros.  A
+// tile whose columns lie in more than one branch takes the branches in turn.
+// Same MFMAs in the same order as lora_blocks.  `buf` holds (BM + BN) * 256
+// bytes that nothing else uses; the caller has a barrier behind it, and the
+// function ends with one.
+template <int BM, int BN, int WGM, int WGN>
+__device__ __forceinline__ void lora_blocks_lds(const GemmParams& p, int64_t m0, int64_t n0, int wm,
+                                                int wn, int wave, int lane, const uint8_t* buf,
+                                                uint32_t buf_lds, v16f* d) {
+  constexpr int WM = BM / WGM, WN = BN / WGN, MB = WM / 32, NB = WN / 32, RS = 8, PITCH = 256;
+  constexpr int WAVES = WGM * WGN, DT = BM / 4 / WAVES, DB = BN / 4 / WAVES;  // 1 KB = 4 rows
+  static_assert(BM % (16 * WAVES) == 0 && BN % (16 * WAVES) == 0, "whole swizzle periods per wave");
+  const int fr = lane & 31, fh = lane >> 5;
+  const int64_t rows_a = min((int64_t)BM, p.m - m0), rows_b = min((int64_t)BN, p.n - n0);
+  const uint32_t row_end = (uint32_t)((p.rank + 7) / 8 * 16);  // bytes of a row that are read
+  auto stage = [&](const uint16_t* base, int64_t ld, int64_t rows, uint32_t dst, auto count) {
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(base, (uint32_t)((rows - 1) * ld * 2) + row_end);
+    static_for<count>([&](auto i) {
+      const int row = (wave * count + i) * 4 + (lane >> 4);
+      const uint32_t chunk = (uint32_t)((lane & 15) ^ (row & 15)) * 16u;
+      const bool ok = row < rows && chunk < row_end;
+      lds_dma16(r, dst + (uint32_t)(wave * count + i) * 1024u,
+                ok ? (uint32_t)row * (uint32_t)(ld * 2) + chunk : VFA_OOB);
+    });
+  };
+  // A fragment of rank step st: positions at or past the rank as zeros.
+  auto frag = [&](const uint8_t* rows, int row, auto st) {
+    v8s v = *reinterpret_cast<const v8s*>(rows + row * PITCH + (((2 * st + fh) ^ (row & 15)) << 4));
+    if (p.rank & 7) {  // uniform: only ranks that end inside an 8-element chunk
+      const int valid = p.rank - (st * 16 + fh * 8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e >= valid) v[e] = 0;
+    }
+    return v;
+  };
+  const int64_t bc = p.lora_branch_cols;
+  auto branch_of = [&](int64_t col) {
+    return __builtin_amdgcn_readfirstlane(bc > 0 ? (int)(col >= bc) + (int)(col >= 2 * bc) : 0);
+  };
+  const int first = branch_of(n0), last = branch_of(min(n0 + BN, p.n) - 1);
+  stage(p.lora_b + n0 * p.ldb, p.ldb, rows_b, buf_lds + BM * PITCH, std::integral_constant<int, DB>{});
+  for (int b = first; b <= last; ++b) {
+    stage(p.lora_t + m0 * p.ldt + b * p.lora_t_branch, p.ldt, rows_a, buf_lds,
+          std::integral_constant<int, DT>{});
+    wait_vmcnt<0, true>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    static_for<NB>([&](auto nb) {
+      const int col = wn * WN + nb * 32;
+      if (branch_of(min(n0 + col, p.n - 1)) == b) {
+        v8s bf[RS];
+        static_for<RS>([&](auto st) { bf[st] = frag(buf + BM * PITCH, col + fr, st); });
+        static_for<MB>([&](auto mb) {
+          v16f acc = v16f{};
+          static_for<RS>([&](auto st) {
+            if (st * 16 < p.rank)
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  __builtin_bit_cast(v8bf, bf[st]),
+                  __builtin_bit_cast(v8bf, frag(buf, wm * WM + mb * 32 + fr, st)), acc, 0, 0, 0);
+          });
+          d[nb * MB + mb] = acc;
+        });
+      }
+    });
+    // Every wave has read t before the next branch, or the output, overwrites it.
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
 }
 
 // LDS bytes of the staged tile vectors: weight scales (or the one scalar),
@@ -265,9 +343,14 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p,
   static_assert(CH % SWZ == 0 && (SWZ & (SWZ - 1)) == 0, "swizzle stays inside the row");
   constexpr int PITCH = SBN * 2;
   const int lane = tid & 63, fr = lane & 31, fh = lane >> 5;
-  const LoraBranch br =
-      LORA ? lora_branch(p, tile_column<BN, SWIGLU>(p, n0, block_col<BN, WN, SWIGLU>(wn, 0)))
-           : LoraBranch{0, 1.0f};
+  // The branch of each column block: one for the whole wave, except in tiles
+  // whose wave width (96) may not divide the branch width.
+  constexpr int BRANCHES = LORA && (WN & (WN - 1)) ? NB : 1;
+  LoraBranch branch[BRANCHES];
+  static_for<BRANCHES>([&](auto nb) {
+    branch[nb] = LORA ? lora_branch(p, tile_column<BN, SWIGLU>(p, n0, block_col<BN, WN, SWIGLU>(wn, nb)))
+                      : LoraBranch{0, 1.0f};
+  });
   const float* __restrict__ sa_p = p.sa;
   const float* __restrict__ sw_p = p.sw;
   const uint16_t* __restrict__ bias_p = p.bias;
@@ -296,6 +379,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p,
   auto lora_delta = [&](auto nb, auto mb) {
     v16f d = v16f{};
     if constexpr (LORA) {
+      const LoraBranch& br = branch[BRANCHES > 1 ? (int)nb : 0];
       if (lora_d) {
         d = lora_d[nb * MB + mb];
       } else {
