@@ -11,9 +11,9 @@ pytestmark = pytest.mark.gpu
 
 
 # On 256 CUs: 4100 rows of rank 48 and 100 take 2x4 blocks (partial row and rank
-# groups), 4100 rows of rank 500 and 32761 of 48 take 4x4.  K = 72 leaves chunks
-# empty, 264 and 1032 end inside a 32-element step.
-@pytest.mark.parametrize("m,rank,k", [(4100, 48, 264), (4100, 100, 72), (4100, 500, 72), (32761, 48, 1032)])
+# groups), 4100 rows of rank 500 and 32761 of 48 take 4x4.  K = 80 leaves chunks
+# empty, and every K here ends inside a 32-element step.
+@pytest.mark.parametrize("m,rank,k", [(4100, 48, 272), (4100, 100, 80), (4100, 500, 80), (32761, 48, 1040)])
 def test_blocks_agree_bit_for_bit(dev, m, rank, k):
     g = torch.Generator(device=dev).manual_seed(m + rank)
     x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)

@@ -119,6 +119,19 @@ def library() -> ctypes.CDLL:
     return lib
 
 
+@cache
+def host():
+    """The native host path (csrc/host.cpp), built next to the library."""
+    library()
+    try:
+        from vflash_amd import _host
+    except ImportError as e:
+        raise RuntimeError(
+            "vflash_amd/_host.so is not built for this Python and torch; run `python -m vflash_amd.build`"
+        ) from e
+    return _host
+
+
 def call(name: str, *args) -> None:
     """Invoke an entry point; map a negative status to an exception."""
     status = getattr(library(), name)(*args)

@@ -2,7 +2,8 @@
 
 Usage: ``python -m vflash_amd.build`` (or ``build()`` from Python).  Each
 ``csrc/*.hip`` file compiles to an object in parallel, then one shared library
-is linked next to this file, where :mod:`vflash_amd._lib` loads it.
+is linked next to this file, where :mod:`vflash_amd._lib` loads it, and the native
+host path (``csrc/host.cpp``, ``_host.so``) against it.
 """
 
 from __future__ import annotations
@@ -12,6 +13,7 @@ import os
 import struct
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from decimal import Decimal, localcontext
 from fractions import Fraction
@@ -20,6 +22,7 @@ from pathlib import Path
 PACKAGE = Path(__file__).resolve().parent
 CSRC = PACKAGE / "csrc"
 LIBRARY = PACKAGE / "libvflash_amd.so"
+HOST_MODULE = PACKAGE / "_host.so"
 OBJECTS = PACKAGE / "_objects"
 ARCH = "gfx950"
 
@@ -220,6 +223,30 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def build_host() -> Path:
+    """Compile csrc/host.cpp, the native host path (a CPython module on torch's C++
+    API), against the built C-ABI library that sits beside it."""
+    import torch
+    from torch.utils import cpp_extension
+
+    source, obj, tmp = CSRC / "host.cpp", OBJECTS / "host.o", HOST_MODULE.with_suffix(".so.tmp")
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    defines = ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    libraries = [f"-L{p}" for p in cpp_extension.library_paths()]
+    for cmd in (
+        [hipcc(), "-x", "c++", "-std=c++20", "-O2", "-fPIC", "-w", *defines,
+         *(arg for p in includes for arg in ("-isystem", p)), "-c", str(source), "-o", str(obj)],
+        ["g++", "-shared", str(obj), f"-L{PACKAGE}", "-lvflash_amd", *libraries, "-lc10", "-lc10_hip", "-ltorch_cpu",
+         "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN", "-o", str(tmp)],
+    ):
+        result = subprocess.run(cmd, capture_output=True, text=True)
+        if result.returncode != 0:
+            raise RuntimeError(f"building {source.name} failed:\n{result.stderr}")
+    os.replace(tmp, HOST_MODULE)
+    return HOST_MODULE
+
+
 def build(verbose: bool = False) -> Path:
     """Compile every HIP source for gfx950 and link the C-ABI library."""
     OBJECTS.mkdir(exist_ok=True)
@@ -237,6 +264,7 @@ def build(verbose: bool = False) -> Path:
     if result.returncode != 0:
         raise RuntimeError(f"link failed:\n{result.stderr}")
     os.replace(tmp, LIBRARY)
+    build_host()
     if verbose:
         print(f"built {LIBRARY}", file=sys.stderr)
     return LIBRARY

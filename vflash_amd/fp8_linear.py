@@ -56,6 +56,11 @@ def _quantize_activation_torch(matrix):
     return codes, act_scale
 
 
+def _unmeasured(_name: str) -> AbstractContextManager[Any]:
+    """The ``measure`` of an execution that none was given to."""
+    return nullcontext()
+
+
 def w8a8_supported(value: torch.Tensor) -> bool:
     return value.dtype == torch.bfloat16 and _lib.is_gfx950(value.device)
 
@@ -85,7 +90,7 @@ class RowFP8Execution:
             raise ValueError("fast_accum must be an explicit boolean")
         self.activation_quantizer = activation_quantizer
         self.fast_accum = fast_accum
-        self.measure = measure if measure is not None else lambda _name: nullcontext()
+        self.measure = measure if measure is not None else _unmeasured
         self.observer: Callable[[], None] | None = None
         self.calls = {"weight_only": 0, "w8a8": 0}
         self.select(mode)
@@ -95,9 +100,26 @@ class RowFP8Execution:
             raise ValueError("unknown FP8 execution mode")
         self.mode = mode
 
+    def native(self, value) -> bool:
+        """Whether a call may run through the native host path: W8A8 with the HIP
+        quantizer, no scope to open between its kernels, a tensor on a GPU."""
+        return (
+            self.mode == "w8a8"
+            and self.activation_quantizer != "torch"
+            and self.measure is _unmeasured
+            and isinstance(value, torch.Tensor)
+            and value.is_cuda
+        )
+
     def linear(self, value, weight, scale, bias=None):
         if self.observer is not None and sum(self.calls.values()) % 200 == 0:
             self.observer()
+        if self.native(value):
+            # The whole call in native code; None sends any other layout on from here.
+            output = _lib.host().w8a8_linear(value, weight, scale, bias)
+            if output is not None:
+                self.calls["w8a8"] += 1
+                return output
         if (
             weight.ndim != 2
             or value.ndim < 1
