@@ -87,11 +87,13 @@ PyObject* w8a8_linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   int status;
   {
     const NoGil nogil;
-    // Codes, then scales, in one allocation (a whole number of 256-byte runs of codes).
-    const at::Tensor work = at::empty({l.m_pad * (l.k + 4)}, l.x->options().dtype(at::kByte));
+    // Two allocations: with the scales right behind the codes (a whole number of
+    // megabytes away) the 4096x3072x3072 linear took 43.8 us instead of 42.9.
+    const at::Tensor code_rows = at::empty({l.m_pad, l.k}, l.x->options().dtype(at::kByte));
+    const at::Tensor row_scales = at::empty({l.m_pad}, l.x->options().dtype(at::kFloat));
     out = output(l);
-    uint8_t* codes = static_cast<uint8_t*>(work.data_ptr());
-    float* scales = reinterpret_cast<float*>(codes + l.m_pad * l.k);
+    uint8_t* codes = static_cast<uint8_t*>(code_rows.data_ptr());
+    float* scales = static_cast<float*>(row_scales.data_ptr());
     void* stream = c10::hip::getCurrentHIPStream(l.x->device().index()).stream();
     status = vflash_quantize_rows_e4m3(l.x->data_ptr(), l.m, l.k, l.k, codes, scales, l.m_pad, stream);
     if (status == VFLASH_OK)
@@ -130,13 +132,13 @@ PyObject* w8a8_linear_lora(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   int status;
   {
     const NoGil nogil;
-    // Codes, scales, t (each starts on a 64-byte boundary).
-    const at::Tensor work =
-        at::empty({l.m_pad * (l.k + 4) + l.m * ldt * 2}, l.x->options().dtype(at::kByte));
+    const at::Tensor code_rows = at::empty({l.m_pad, l.k}, l.x->options().dtype(at::kByte));
+    const at::Tensor row_scales = at::empty({l.m_pad}, l.x->options().dtype(at::kFloat));
+    const at::Tensor t_rows = at::empty({l.m, ldt}, l.x->options());
     out = output(l);
-    uint8_t* codes = static_cast<uint8_t*>(work.data_ptr());
-    float* scales = reinterpret_cast<float*>(codes + l.m_pad * l.k);
-    void* t = scales + l.m_pad;
+    uint8_t* codes = static_cast<uint8_t*>(code_rows.data_ptr());
+    float* scales = static_cast<float*>(row_scales.data_ptr());
+    void* t = t_rows.data_ptr();
     void* stream = c10::hip::getCurrentHIPStream(l.x->device().index()).stream();
     status = vflash_quantize_rows_lora_e4m3(l.x->data_ptr(), l.m, l.k, l.k, codes, scales, l.m_pad,
                                             down->data_ptr(), rank, t, ldt, stream);
