@@ -33,7 +33,7 @@ def check(out, x, codes, scale, bias):
 
 
 # Partial tiles in rows and columns, K tails inside a 64-K stage, each tiling
-# (64x64; 128x64 at 200 x 5128; 128x128 at 600 x 5128; 256x128 at 1000 x 7176)
+# (64x64; 128x64 at 200 x 5128; 128x128 at 600 x 5128; 128x256 at 1000 x 7176)
 # and the restoring pass (1025 rows).
 @pytest.mark.parametrize("m,k,n", [(1, 16, 8), (17, 48, 272), (65, 144, 72), (200, 80, 5128),
                                    (600, 208, 5128), (1000, 272, 7176), (1025, 112, 136)])

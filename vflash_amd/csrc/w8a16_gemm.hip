@@ -34,20 +34,22 @@ struct W16Layout {
   static constexpr int PER_CU = 2 * (RING + VEC_LDS) <= 160 * 1024 ? 2 : 1;
 };
 
-template <int BM, int BN, int NS>
+template <int BM, int BN, int NS, int WGM>
 __global__ void __launch_bounds__(256, (W16Layout<BM, BN, NS>::PER_CU)) w8a16_gemm_pipe(
     const GemmParams p) {
   using L = W16Layout<BM, BN, NS>;
-  static_assert(BM % 64 == 0 && BN % 64 == 0 && NS % 2 == 0 && (NS - 1) * L::DMA < 64, "tiling");
+  constexpr int WGN = 4 / WGM;
+  static_assert(BM % (32 * WGM) == 0 && BN % (32 * WGN) == 0 && BM % 64 == 0 && BN % 64 == 0 &&
+                NS % 2 == 0 && (NS - 1) * L::DMA < 64, "tiling");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[L::RING];
   __shared__ __attribute__((aligned(1024))) uint8_t vec[VEC_LDS];
-  constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 32, NB = WN / 32;
+  constexpr int WM = BM / WGM, WN = BN / WGN, MB = WM / 32, NB = WN / 32;
   int tm, tn;
   tile_coords((int)((p.m + BM - 1) / BM), (int)((p.n + BN - 1) / BN), p.group_m, tm, tn);
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = (int)threadIdx.x & 63;
   const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_addr(ring));
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WGM, wn = wave / WGM;
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const int64_t rows_a = min((int64_t)BM, p.m - m0), rows_w = min((int64_t)BN, p.n - n0);
   // p.lda counts bytes here as everywhere; resources end with the tile's last
@@ -190,22 +192,24 @@ __global__ void __launch_bounds__(256, (W16Layout<BM, BN, NS>::PER_CU)) w8a16_ge
   wait_vmcnt<0, true>();  // every DMA has landed before the ring becomes the staging tile
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  gemm_epilogue<BM, BN, 2, 2, EPI_LINEAR, true>(p, acc, m0, n0, wm, wn, (int)threadIdx.x, ring, vec);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI_LINEAR, true>(p, acc, m0, n0, wm, wn, (int)threadIdx.x, ring, vec);
 }
 
 int compute_units();
 
-template <int BM, int BN, int NS>
+template <int BM, int BN, int NS, int WGM>
 static void launch_w16(const GemmParams& p, hipStream_t s) {
   const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
-  w8a16_gemm_pipe<BM, BN, NS><<<dim3((unsigned)tiles), dim3(256), 0, s>>>(p);
+  w8a16_gemm_pipe<BM, BN, NS, WGM><<<dim3((unsigned)tiles), dim3(256), 0, s>>>(p);
 }
 
 // The tiling, as in the NVFP4 GEMM: the least estimated time of the busiest CU
 // (microseconds at K = 5120; a first tile, and each further one).  Measured at
-// N = 5120 as 64x64, 128x64, 128x128 and 256x128: M = 16 26.3, 31.7, 46.2, 67.4;
-// M = 200 38.7, 32.9, 46.8, 68.5; M = 512 60.6, 63.0, 48.9, 69.5; 1024 x 5376 x
-// 7168 143.7, 136.8, 95.5, 85.5.
+// N = 5120 as 64x64, 128x64, 128x128 and 128x256: M = 17 26.7, 31.6, 41.1, 63.0;
+// M = 200 38.9, 33.5, 43.3, 63.3; M = 512 60.3, 64.5, 44.9, 65.4; M = 1024 98.7,
+// 96.9, 89.2, 67.5.  The two widest put their four waves side by side, so that no
+// weight fragment is converted twice (2x2 waves: M = 512 50.3, 1024 x 7168 as
+// 256x128 83.1 against 81.9).
 hipError_t launch_w8a16(const GemmParams& params, hipStream_t s) {
   GemmParams p = params;
   p.group_m = 8;
@@ -214,16 +218,16 @@ hipError_t launch_w8a16(const GemmParams& params, hipStream_t s) {
     const int64_t tiles = ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn);
     return first + more * ((tiles + cus - 1) / cus - 1);
   };
-  const int64_t c[4] = {cost(256, 128, 72, 75), cost(128, 128, 46, 44), cost(128, 64, 31, 31),
-                        cost(64, 64, 26, 15)};
+  const int64_t c[4] = {cost(128, 256, 66, 77), cost(128, 128, 45, 46), cost(128, 64, 32, 32),
+                        cost(64, 64, 27, 14)};
   int best = 0;
   for (int t = 1; t < 4; ++t)
     if (c[t] < c[best]) best = t;
   switch (best) {
-    case 0: launch_w16<256, 128, 2>(p, s); break;
-    case 1: launch_w16<128, 128, 2>(p, s); break;
-    case 2: launch_w16<128, 64, 6>(p, s); break;
-    default: launch_w16<64, 64, 6>(p, s); break;
+    case 0: launch_w16<128, 256, 4, 1>(p, s); break;
+    case 1: launch_w16<128, 128, 4, 1>(p, s); break;
+    case 2: launch_w16<128, 64, 6, 2>(p, s); break;
+    default: launch_w16<64, 64, 6, 2>(p, s); break;
   }
   return hipGetLastError();
 }
