@@ -154,9 +154,9 @@ int64_t vflash_swiglu_parts(int64_t n);
  * m x n output on a device with `compute_units` CUs (a host-side query; no
  * device work).  0: 256x256, 1: 256x192, 2: 256x128, 3: 128x192, 4: 128x128
  * (two workgroups per CU), 5: 128x128 (one per CU, grids of one round),
- * 6: 128x64, 7: 64x64.  The SwiGLU entries always use 256x256.  The plain and
- * gate-residual entries may run 256x256 tiles with a last round of smaller ones
- * where this answers 256x256 or 256x192.  No tiling
+ * 6: 128x64, 7: 64x64.  The SwiGLU entries use 256x256 (64x256 in a nearly
+ * empty last round).  The plain and gate-residual entries may run 256x256 tiles with
+ * a last round of smaller ones where this answers 256x256 or 256x192.  No tiling
  * changes a result bit; this exists so that tests can aim shapes at each one.
  * branch_cols > 0 (a multiple of 32): the choice of a LoRA entry with adapter
  * branches that wide: the best of the tilings whose wave width (half the tile width)
@@ -403,6 +403,13 @@ int vflash_nvfp4_linear(const void* a, const float* sa, int64_t lda, const void*
 int vflash_nvfp4_quantize_rows(const void* x, int x_is_f16, int64_t m, int64_t k, int64_t ldx,
                                const float* global_sf, void* codes, int64_t ldc, void* scales,
                                int64_t m_pad, void* stream);
+
+/* The same, and out_scale[0] = alpha[0] / global_sf[0] (one binary32 division), the output scale
+ * of the W4A4 linear that consumes the rows, without a launch of its own. */
+int vflash_nvfp4_quantize_rows_scaled(const void* x, int x_is_f16, int64_t m, int64_t k, int64_t ldx,
+                                      const float* global_sf, void* codes, int64_t ldc, void* scales,
+                                      int64_t m_pad, const float* alpha, float* out_scale,
+                                      void* stream);
 
 /*
  * W4A4 NVFP4 linear: E2M1 activations and weights, each with E4M3 scales per

@@ -35,3 +35,15 @@ def test_tilings_agree_bit_for_bit(dev, k, activations):
     whole = linear(x)
     for m in (1, 17, 65, 300, 1000, 2047, 4001):
         assert torch.equal(linear(x[:m]), whole[:m]), m
+
+
+@pytest.mark.parametrize("m,k", [(1, 64), (300, 512)])
+def test_output_scale_of_the_quantizer_is_the_device_division(dev, m, k):
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
+    for a, b in ((0.0123, 487.3), (3.0, 0.1), (1e-38, 3e5), (float("inf"), 2.0)):
+        alpha, gsf = torch.tensor(a, device=dev), torch.tensor(b, device=dev)
+        codes, scales, out_scale = kernels.nvfp4_quantize_rows(x, gsf, alpha)
+        plain_codes, plain_scales = kernels.nvfp4_quantize_rows(x, gsf)
+        assert torch.equal(out_scale, alpha / gsf)
+        assert torch.equal(codes, plain_codes) and torch.equal(scales, plain_scales)

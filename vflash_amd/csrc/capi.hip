@@ -25,7 +25,7 @@ hipError_t launch_lora_down(const uint16_t*, int64_t, int64_t, int64_t, const ui
 hipError_t launch_quant_lora(const uint16_t*, int64_t, int64_t, int64_t, const uint16_t*, int,
                              uint16_t*, int64_t, uint8_t*, float*, int64_t, hipStream_t);
 hipError_t launch_nvfp4_quant(const uint16_t*, bool, int64_t, int64_t, int64_t, const float*,
-                              uint8_t*, int64_t, uint8_t*, int64_t, hipStream_t);
+                              uint8_t*, int64_t, uint8_t*, int64_t, const float*, float*, hipStream_t);
 hipError_t launch_nvfp4_w4a4(const uint8_t*, int64_t, const uint8_t*, const uint8_t*,
                              const uint8_t*, const float*, int64_t, int64_t, int64_t,
                              const uint16_t*, uint16_t*, int64_t, int, hipStream_t);
@@ -429,14 +429,23 @@ int vflash_nvfp4_linear(const void* a, const float* sa, int64_t lda, const void*
 int vflash_nvfp4_quantize_rows(const void* x, int x_is_f16, int64_t m, int64_t k, int64_t ldx,
                                const float* global_sf, void* codes, int64_t ldc, void* scales,
                                int64_t m_pad, void* stream) {
+  return vflash_nvfp4_quantize_rows_scaled(x, x_is_f16, m, k, ldx, global_sf, codes, ldc, scales, m_pad,
+                                           nullptr, nullptr, stream);
+}
+
+int vflash_nvfp4_quantize_rows_scaled(const void* x, int x_is_f16, int64_t m, int64_t k, int64_t ldx,
+                                      const float* global_sf, void* codes, int64_t ldc, void* scales,
+                                      int64_t m_pad, const float* alpha, float* out_scale,
+                                      void* stream) {
   if (!x || !global_sf || !codes || !scales || m < 1 || k < 64 || k % 64) return VFLASH_EINVAL;
   if (ldx < k || ldx % 8 || ldc < k / 2 || ldc % 16 || m_pad < m || m_pad % 128) return VFLASH_EINVAL;
   if (m_pad >= (int64_t(1) << 33)) return VFLASH_EINVAL;
   if (!aligned(x, 16) || !aligned(codes, 16) || !aligned(scales, 4) || !aligned(global_sf, 4))
     return VFLASH_EINVAL;
+  if (!alpha != !out_scale || !aligned(alpha, 4) || !aligned(out_scale, 4)) return VFLASH_EINVAL;
   return status(vfa::launch_nvfp4_quant(static_cast<const uint16_t*>(x), x_is_f16 != 0, m, k, ldx,
                                         global_sf, static_cast<uint8_t*>(codes), ldc,
-                                        static_cast<uint8_t*>(scales), m_pad,
+                                        static_cast<uint8_t*>(scales), m_pad, alpha, out_scale,
                                         static_cast<hipStream_t>(stream)));
 }
 

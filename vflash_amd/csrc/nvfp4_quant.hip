@@ -45,7 +45,12 @@ __global__ void __launch_bounds__(256) nvfp4_quant_rows(const uint16_t* __restri
                                                         const float* __restrict__ global_sf,
                                                         uint8_t* __restrict__ codes, int64_t ldc,
                                                         uint8_t* __restrict__ scales,
-                                                        int64_t m_pad) {
+                                                        int64_t m_pad,
+                                                        const float* __restrict__ alpha,
+                                                        float* __restrict__ out_scale) {
+  // The GEMM's output scale, one IEEE division, for the launch that follows.
+  if (out_scale && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
+    *out_scale = *alpha / *global_sf;
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= m_pad) return;
@@ -111,12 +116,15 @@ unsigned row_segments(int64_t rows, int64_t k);
 
 hipError_t launch_nvfp4_quant(const uint16_t* x, bool f16, int64_t m, int64_t k, int64_t ldx,
                               const float* global_sf, uint8_t* codes, int64_t ldc,
-                              uint8_t* scales, int64_t m_pad, hipStream_t s) {
+                              uint8_t* scales, int64_t m_pad, const float* alpha, float* out_scale,
+                              hipStream_t s) {
   const dim3 grid((unsigned)((m_pad + 3) / 4), row_segments(m_pad, k));
   if (f16)
-    nvfp4_quant_rows<true><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad);
+    nvfp4_quant_rows<true><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad,
+                                        alpha, out_scale);
   else
-    nvfp4_quant_rows<false><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad);
+    nvfp4_quant_rows<false><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad,
+                                        alpha, out_scale);
   return hipGetLastError();
 }
 

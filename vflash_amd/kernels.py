@@ -572,13 +572,14 @@ def nvfp4_gemm(codes, act_scale, packed, block_scales, alpha, rows, bias=None):
     return out
 
 
-def nvfp4_quantize_rows(matrix, global_sf):
+def nvfp4_quantize_rows(matrix, global_sf, alpha=None):
     """NVFP4 activation quantization (the W4A4 input).
 
     ``matrix`` is bf16 or f16 ``[M, K]`` (K % 64 == 0, unit column stride),
     ``global_sf`` an fp32 scalar tensor on the same device.  Returns packed E2M1
     codes ``[M, K/2]`` (uint8) and E4M3 block scales ``[ceil128(M), K/16]``
-    (uint8, 128x4 order, padding rows 0).
+    (uint8, 128x4 order, padding rows 0).  With ``alpha`` (an fp32 scalar tensor)
+    also the output scale ``alpha / global_sf``, formed in the same launch.
     """
     if matrix.dtype not in (torch.bfloat16, torch.float16) or matrix.ndim != 2 or matrix.stride(1) != 1:
         raise ValueError("NVFP4 quantization requires a 2-D BF16/F16 matrix with unit column stride")
@@ -591,11 +592,19 @@ def nvfp4_quantize_rows(matrix, global_sf):
     m_pad = (m + 127) // 128 * 128
     codes = torch.empty((m, k // 2), device=device, dtype=torch.uint8)
     scales = torch.empty((m_pad, k // 16), device=device, dtype=torch.uint8)
-    if m:
-        call("vflash_nvfp4_quantize_rows", ptr(matrix), int(matrix.dtype == torch.float16), m, k,
-             matrix.stride(0), ptr(global_sf), ptr(codes), codes.stride(0), ptr(scales), m_pad,
-             stream_of(device))
-    return codes, scales
+    if alpha is None:
+        if m:
+            call("vflash_nvfp4_quantize_rows", ptr(matrix), int(matrix.dtype == torch.float16), m, k,
+                 matrix.stride(0), ptr(global_sf), ptr(codes), codes.stride(0), ptr(scales), m_pad,
+                 stream_of(device))
+        return codes, scales
+    if alpha.dtype != torch.float32 or alpha.numel() != 1 or alpha.device != device or not m:
+        raise ValueError("the NVFP4 output scale needs an fp32 alpha on the rows' device")
+    out_scale = torch.empty((), device=device, dtype=torch.float32)
+    call("vflash_nvfp4_quantize_rows_scaled", ptr(matrix), int(matrix.dtype == torch.float16), m, k,
+         matrix.stride(0), ptr(global_sf), ptr(codes), codes.stride(0), ptr(scales), m_pad,
+         ptr(alpha), ptr(out_scale), stream_of(device))
+    return codes, scales, out_scale
 
 
 def nvfp4_w4a4_gemm(codes, act_scales, packed, block_scales, alpha, rows, bias=None):

@@ -117,9 +117,8 @@ class NVFP4Execution:
         if self.activations == "nvfp4":
             if matrix.data_ptr() % 16:
                 matrix = matrix.clone()  # the quantizer reads 16-byte vectors
-            codes, scales = kernels.nvfp4_quantize_rows(matrix, weight.input_scale)
             # The output scale as the reference forms it (one fp32 division on the device).
-            alpha = weight.alpha / weight.input_scale
+            codes, scales, alpha = kernels.nvfp4_quantize_rows(matrix, weight.input_scale, weight.alpha)
             output = kernels.nvfp4_w4a4_gemm(
                 codes, scales, weight.packed, weight.scales, alpha, matrix.shape[0], bias
             )
