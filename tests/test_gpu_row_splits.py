@@ -42,3 +42,25 @@ def test_few_rows_match_many(dev, k):
         tiles = (m + 127) // 128
         assert torch.equal(c, f_codes[:m]), m
         assert torch.equal(s.reshape(tiles, -1), whole.reshape(-1, s.numel() // tiles)[:tiles]), m
+
+
+# 3000 rows take one wave a row on 256 CUs; 1, 17 and 700 four, 1500 two, and
+# 4095 (two rounds of whole rows) two.
+@pytest.mark.parametrize("k", [8, 520, 4104, 13824, 16384])
+def test_gelu_rows_shared_between_waves(dev, k):
+    g = torch.Generator(device=dev).manual_seed(k)
+    y = (torch.randn((4095, k), generator=g, device=dev) * 2).to(torch.bfloat16)
+    y[3, k - 1] = float("nan")
+    y[4, k // 2] = float("inf")
+    y[6] = 0
+    bits = lambda t: t.contiguous().view(torch.uint8)
+    codes, scales, values = kernels.gelu_quantize_rows(y[:3000], keep_values=True)
+    for m in (1, 17, 700, 1500, 4095):
+        c, s, v = kernels.gelu_quantize_rows(y[:m], keep_values=True)
+        n = min(m, 3000)
+        assert torch.equal(bits(c[:n]), bits(codes[:n])) and torch.equal(bits(s[:n]), bits(scales[:n])), m
+        assert torch.equal(bits(v[:n]), bits(values[:n])), m
+        assert not c[m:].view(torch.uint8).any() and bool((s[m:] == 1).all()), m
+    c, s, v = kernels.gelu_quantize_rows(y[3000:], keep_values=True)
+    whole = kernels.gelu_quantize_rows(y, keep_values=True)
+    assert torch.equal(bits(whole[0][3000:4095]), bits(c[:1095])) and torch.equal(bits(whole[2][3000:]), bits(v))

@@ -29,6 +29,7 @@
 namespace vfa {
 
 extern template hipError_t launch_mixed<EPI_BIAS>(const GemmParams&, int64_t, int, hipStream_t);
+extern template hipError_t launch_mixed<EPI_SWIGLU>(const GemmParams&, int64_t, int, hipStream_t);
 extern template hipError_t launch_mixed<EPI_GATE>(const GemmParams&, int64_t, int, hipStream_t);
 extern template hipError_t launch_tiling<EPI_BIAS>(const GemmParams&, int, hipStream_t);
 extern template hipError_t launch_tiling<EPI_GATE>(const GemmParams&, int, hipStream_t);
@@ -131,6 +132,29 @@ static int mixed_tail(const GemmParams& p, int tiling, int64_t tiles, int64_t cu
   return tiling == GEMM_256x192 && 4 * rem <= cus ? MIXED_128x128 : MIXED_NONE;
 }
 
+// SwiGLU: the 256x256 tiles that run whole when the rest runs as 64x256 tiles, or
+// -1 where splitting does not pay: only while the 64x256 tiles fit one round.
+// Microseconds whole and split at K 5376, F 14336: 9 rows 52.4, 44.8; 100 rows
+// 55.0, 48.6; 1100 179, 155 (two rounds and 48 tiles); 3000 382, 356; at 300 x 2048
+// x 4096 28.8, 15.1.  With more than a round of them: 300 rows 59.3, 91.7; 777
+// rows 127, 140; 1024 131, 149.
+static int64_t swiglu_main_tiles(const GemmParams& p, int64_t cus) {
+  if (p.k % 128) return -1;
+  const int64_t tiles_m = (p.m + 255) / 256, tiles_n = p.half_n / 128, tiles = tiles_m * tiles_n;
+  const int64_t main = tiles / cus * cus;
+  if (tiles == main || main >= 8 * cus) return -1;
+  // 64-row tiles of the last round that hold any row (grouped_tile's order).
+  int64_t live = 0;
+  for (int64_t t = main; t < tiles; ++t) {
+    const int64_t group = t / (p.group_m * tiles_n), first = group * p.group_m;
+    const int64_t rows = tiles_m - first < p.group_m ? tiles_m - first : p.group_m;
+    const int64_t tm = first + (t - group * p.group_m * tiles_n) % rows;
+    const int64_t left = (p.m - tm * 256 + 63) / 64;
+    live += left < 4 ? left : 4;
+  }
+  return live <= cus ? main : -1;
+}
+
 // GemmParams::group_m is set here from the tiling.
 hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
   GemmParams p = params;
@@ -138,6 +162,8 @@ hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
     // One tiling: 128 value + 128 gate columns, the 256x256 schedule.
     p.group_m = tiling_group_m(GEMM_256x256, (p.half_n + 127) / 128);
     if (epi == EPI_SWIGLU_LORA) return launch_pipe<EPI_SWIGLU_LORA, PipeCfg<256, 256, SPLIT_RING, 0>>(p, s);
+    const int64_t whole = swiglu_main_tiles(p, compute_units());
+    if (whole >= 0) return launch_mixed<EPI_SWIGLU>(p, whole, MIXED_64x256, s);
     return launch_pipe<EPI_SWIGLU, PipeCfg<256, 256, SPLIT_RING, 0>>(p, s);
   }
   int tiling =

@@ -6,7 +6,7 @@
 
 namespace vfa {
 
-enum { MIXED_NONE = 0, MIXED_256x128 = 1, MIXED_128x128 = 2 };
+enum { MIXED_NONE = 0, MIXED_256x128 = 1, MIXED_128x128 = 2, MIXED_64x256 = 3 };
 
 // A 256x256 grid whose last round would leave most of the CUs idle: the first
 // main_tiles tiles (whole rounds of one tile per CU) run as 256x256, each of the
@@ -15,7 +15,10 @@ enum { MIXED_NONE = 0, MIXED_256x128 = 1, MIXED_128x128 = 2 };
 template <int EPI, int SBM, int SBN, int SNS, int SPRE>
 __global__ void __launch_bounds__(256, 1) fp8_gemm_mixed(const GemmParams p, int main_tiles) {
   constexpr int RING = pipe_lds(256, 256, SPLIT_RING), SRING = pipe_lds(SBM, SBN, SNS);
-  static_assert(SRING + VEC_LDS <= RING && !epi_swiglu(EPI), "the small tile's LDS fits the ring");
+  // SwiGLU tiles are 128 value and 128 gate columns wide, whole or split.
+  static_assert(!epi_swiglu(EPI) || SBN == 256, "value and gate columns stay paired");
+  static_assert(SRING + VEC_LDS + (epi_swiglu(EPI) ? SILU_LDS : 0) <= RING,
+                "the small tile's LDS fits the ring");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[RING];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_addr(ring));
@@ -47,10 +50,11 @@ static hipError_t launch_mixed_as(const GemmParams& p, int64_t main_tiles, hipSt
   return hipGetLastError();
 }
 
-// tail: the tiles of the last round (256x128, or 128x128).
+// tail: the tiles of the last round (256x128 or 128x128; SwiGLU 64x256).
 template <int EPI>
 hipError_t launch_mixed(const GemmParams& p, int64_t main_tiles, int tail, hipStream_t s) {
-  return tail == MIXED_256x128 ? launch_mixed_as<EPI, 256, 128, 3, 0>(p, main_tiles, s)
+  if constexpr (epi_swiglu(EPI)) return launch_mixed_as<EPI, 64, 256, 3, 0>(p, main_tiles, s);
+  else return tail == MIXED_256x128 ? launch_mixed_as<EPI, 256, 128, 3, 0>(p, main_tiles, s)
                                : launch_mixed_as<EPI, 128, 128, 3, -1>(p, main_tiles, s);
 }
 

@@ -104,7 +104,7 @@ __device__ __forceinline__ void pipe_tile(const GemmParams& p, int tm, int tn, u
     // Waves 0-1 load tile rows 0..BN/2-1 = value rows n0.., waves 2-3 load tile
     // rows BN/2.. = gate rows half_n + n0.. (the resource is based BN/2 rows
     // earlier, so tile row r maps to half_n + n0 + r - BN/2).
-    static_assert(BM == 256 && BN == 256 && DMA_W * 8 * 2 == BN / 2,
+    static_assert(BN == 256 && DMA_W * 8 * 2 == BN / 2,
                   "each wave loads rows of one half");
     const int64_t rows_h = min((int64_t)(BN / 2), p.half_n - n0);
     full = full && rows_h == BN / 2;
