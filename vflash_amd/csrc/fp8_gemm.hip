@@ -25,9 +25,14 @@
 // scales, each owning a contiguous run of output columns (the Q/K/V adapters of
 // a merged projection, h3_native_denoiser.py:301-316, h3_fused_ops.py:900-980).
 #include "fp8_gemm_mixed.h"
+#include "fp8_gemm_skinny.h"
 
 namespace vfa {
 
+extern template hipError_t launch_skinny<EPI_BIAS>(const GemmParams&, int, hipStream_t);
+extern template hipError_t launch_skinny<EPI_GATE>(const GemmParams&, int, hipStream_t);
+extern template hipError_t launch_skinny<EPI_LORA>(const GemmParams&, int, hipStream_t);
+extern template hipError_t launch_skinny<EPI_LORA_GATE>(const GemmParams&, int, hipStream_t);
 extern template hipError_t launch_mixed<EPI_BIAS>(const GemmParams&, int64_t, int, hipStream_t);
 extern template hipError_t launch_mixed<EPI_SWIGLU>(const GemmParams&, int64_t, int, hipStream_t);
 extern template hipError_t launch_mixed<EPI_GATE>(const GemmParams&, int64_t, int, hipStream_t);
@@ -155,6 +160,18 @@ static int64_t swiglu_main_tiles(const GemmParams& p, int64_t cus) {
   return live <= cus ? main : -1;
 }
 
+// Rows per workgroup (32 or 64) of the few-row kernel, or 0: the smaller one whose
+// workgroups all get a CU of their own.  Two on a CU share its LDS and L1 and lose
+// what the split of roles gains.  Microseconds, 64x64 tiles -> 32 rows, 64 rows:
+// 17 x 5120 x 5120 11.1 -> 7.6, 8.5; 17 x 14336 x 5376 24.1 -> 14.8, 16.4; 64 x
+// 3072 x 3072 8.8 -> 6.1, 6.6; 64 x 5120 x 5120 12.4 -> 13.4 (320 workgroups), 9.6;
+// 17 x 5120 x 13824 13.4 -> 13.5 (432), 14.5; 128 x 5120 x 5120 12.5 -> 20.4, 15.8.
+static int skinny_rows(const GemmParams& p, int64_t cus) {
+  const int64_t cols = (p.n + 31) / 32;
+  if ((p.m + 31) / 32 * cols <= cus) return 32;
+  return (p.m + 63) / 64 * cols <= cus ? 64 : 0;
+}
+
 // GemmParams::group_m is set here from the tiling.
 hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
   GemmParams p = params;
@@ -165,6 +182,17 @@ hipError_t launch_fp8_gemm(const GemmParams& params, int epi, hipStream_t s) {
     const int64_t whole = swiglu_main_tiles(p, compute_units());
     if (whole >= 0) return launch_mixed<EPI_SWIGLU>(p, whole, MIXED_64x256, s);
     return launch_pipe<EPI_SWIGLU, PipeCfg<256, 256, SPLIT_RING, 0>>(p, s);
+  }
+  const int skinny = skinny_rows(p, compute_units());
+  if (skinny) {
+    p.group_m = 1;
+    switch (epi) {
+      case EPI_BIAS: return launch_skinny<EPI_BIAS>(p, skinny, s);
+      case EPI_GATE: return launch_skinny<EPI_GATE>(p, skinny, s);
+      case EPI_LORA: return launch_skinny<EPI_LORA>(p, skinny, s);
+      case EPI_LORA_GATE: return launch_skinny<EPI_LORA_GATE>(p, skinny, s);
+      default: return hipErrorInvalidValue;
+    }
   }
   int tiling =
       pick_tiling(p.m, p.n, compute_units(), epi_lora(epi) ? p.lora_branch_cols : 0);
