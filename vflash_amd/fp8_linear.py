@@ -13,6 +13,10 @@ package on gfx950 and never falls back to another arithmetic:
 * GEMM + scales + bias: ``vflash_fp8_linear`` with binary32 accumulation and
   the reference's two bf16 roundings (``_scaled_mm`` output, then ``+ bias``).
 
+The weight-only mode is the restored-weight expression of the reference; on gfx950
+its BF16 inference calls run as one GEMM that restores the weight on the fly
+(``kernels.weight_only_linear``), everything else as that torch expression.
+
 ``fast_accum`` is validated and recorded like the reference's; MFMA
 accumulation is always binary32, so it does not change the arithmetic.
 """
