@@ -8,7 +8,7 @@
 // Rows in [m, m_pad) are the GEMM padding rows: codes 0, scale 1.
 //
 // Layout: one 64-lane wave owns one row and a 256-thread workgroup 4 rows, or,
-// with few rows, the workgroup's four waves share one row (WPR = 4).
+// with few or wide rows, the workgroup's four waves share one row (WPR = 4).
 // The aligned kernel keeps the whole row in VGPRs (16-byte loads, one HBM
 // read per element), reduces the maximum across the wave with XOR shuffles and
 // writes 8 codes per 16-byte input vector.
@@ -141,7 +141,10 @@ unsigned row_segments(int64_t rows, int64_t k) {
   return (unsigned)(segs > 1 ? segs : 1);
 }
 
-// Rows up to which the four waves of a workgroup share one row.
+// Rows up to which the four waves of a workgroup share one row at any width.
+// Microseconds unshared -> shared: 300 x 5376 9.5 -> 4.8, 2048 x 5120 11.9 -> 9.1,
+// 32760 x 5120 90 -> 79, 32760 x 14336 387 -> 262, 4095 x 13824 50 -> 33; narrow rows
+// of long calls lose: 4095 x 1536 6.8 -> 7.3, 32760 x 1536 27 -> 38, x 3072 54 -> 55.
 constexpr int64_t QUANT_SHARED_ROWS = 2048;
 
 hipError_t launch_quant_rows(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
@@ -151,9 +154,10 @@ hipError_t launch_quant_rows(const uint16_t* x, int64_t m, int64_t k, int64_t ld
                        ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
                        ((reinterpret_cast<uintptr_t>(codes) & 7) == 0);
   const int64_t nvec = k / 8;
-  if (aligned && nvec <= 64 * 32) {
-    // Few rows: four waves share a row.
-    if (m_pad <= QUANT_SHARED_ROWS && nvec > 64) {
+  if (aligned && nvec <= 64 * 32 && m_pad < (int64_t(1) << 31)) {  // one workgroup per shared row
+    // Four waves share a row when rows are few, and always above 4096 columns,
+    // where one wave's registers for the whole row leave too few waves in flight.
+    if (nvec > 64 && (m_pad <= QUANT_SHARED_ROWS || nvec > 512)) {
       const dim3 rows((unsigned)m_pad);
       if (nvec <= 256) quant_rows_vec<1, 4><<<rows, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
       else if (nvec <= 512) quant_rows_vec<2, 4><<<rows, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
@@ -162,9 +166,7 @@ hipError_t launch_quant_rows(const uint16_t* x, int64_t m, int64_t k, int64_t ld
     } else if (nvec <= 64) quant_rows_vec<1, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
     else if (nvec <= 128) quant_rows_vec<2, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
     else if (nvec <= 256) quant_rows_vec<4, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
-    else if (nvec <= 512) quant_rows_vec<8, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
-    else if (nvec <= 1024) quant_rows_vec<16, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
-    else quant_rows_vec<32, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
+    else quant_rows_vec<8, 1><<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
   } else {
     quant_rows_generic<<<grid, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
   }
