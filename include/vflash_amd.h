@@ -351,7 +351,7 @@ int vflash_fp8_linear_lora_branches(const void* a, const float* sa, int64_t lda,
  *   x    bf16 [m, k] (ldx elements, a multiple of 8); w: E4M3 codes [n, k] (ldw bytes, a
  *        multiple of 16); sw: fp32 [n]; bias: bf16 [n] or NULL; out: bf16 [m, n] (ldo elements,
  *        a multiple of 8); all 16-byte aligned
- *   k a multiple of 16, n a multiple of 8
+ *   k a multiple of 16, n a multiple of 8 below 2^29
  */
 int vflash_w8a16_linear(const void* x, int64_t ldx, const void* w, const float* sw, int64_t ldw,
                         int64_t m, int64_t n, int64_t k, const void* bias, void* out, int64_t ldo,

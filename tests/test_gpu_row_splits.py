@@ -66,3 +66,28 @@ def test_gelu_rows_shared_between_waves(dev, k):
     c, s, v = kernels.gelu_quantize_rows(y[3000:], keep_values=True)
     whole = kernels.gelu_quantize_rows(y, keep_values=True)
     assert torch.equal(bits(whole[0][3000:4095]), bits(c[:1095])) and torch.equal(bits(whole[2][3000:]), bits(v))
+
+
+def test_rows_past_one_grid_dimension(dev):
+    # A workgroup per row: rows past 2^22 start in the grid's second dimension, and
+    # the last workgroups of that one lie past the end.
+    from vflash_amd._lib import call, ptr, stream_of
+
+    n, k = 2**22 + 5, 16
+    g = torch.Generator(device=dev).manual_seed(0)
+    codes = torch.randint(0, 127, (n, k), generator=g, device=dev, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    scale = torch.rand((n, 1), generator=g, device=dev)
+    out = torch.zeros((n + 3, k), device=dev, dtype=torch.bfloat16)
+    call("vflash_restore_rows_bf16", ptr(codes), ptr(scale), k, n, k, ptr(out), stream_of(dev))
+    assert torch.equal(out[:n], (codes.float() * scale).to(torch.bfloat16)) and not out[n:].any()
+    k = 4104  # 34 GB of rows, of which the first and the last few are not zero
+    x = torch.zeros((n, k), device=dev, dtype=torch.bfloat16)
+    ends = torch.cat([torch.arange(3), torch.arange(n - 9, n)]).to(dev)
+    x[ends] = torch.randn((12, k), generator=g, device=dev).to(torch.bfloat16)
+    codes, scales = kernels.quantize_rows(x)
+    few_codes, few_scales = kernels.quantize_rows(x[ends])
+    assert torch.equal(codes[ends].view(torch.uint8), few_codes[:12].view(torch.uint8))
+    assert torch.equal(scales[ends], few_scales[:12]) and bool((scales[3:n - 9] == 1).all())
+    assert not codes[n:].view(torch.uint8).any() and bool((scales[n:] == 1).all())
+    del x, codes
+    torch.cuda.empty_cache()

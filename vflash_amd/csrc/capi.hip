@@ -393,6 +393,7 @@ int vflash_w8a16_linear(const void* x, int64_t ldx, const void* w, const float* 
       (bias && !aligned(bias, 16)))
     return VFLASH_EINVAL;
   if (512 * ldx >= (int64_t(1) << 31) || 256 * ldw >= (int64_t(1) << 31)) return VFLASH_EINVAL;
+  if (n >= (int64_t(1) << 29)) return VFLASH_EINVAL;  // a grid holds 2^24 tiles, of 64 columns at least
   vfa::GemmParams p = base_params(x, nullptr, 2 * ldx, w, sw, ldw, m, n, k, bias, out, ldo);
   return status(vfa::launch_w8a16(p, static_cast<hipStream_t>(stream)));
 }

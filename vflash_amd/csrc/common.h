@@ -22,6 +22,17 @@ __device__ __forceinline__ void static_for(F&& f) {
   }(std::make_integer_sequence<int, N>{});
 }
 
+// One workgroup per row, for any number of rows: HIP takes a grid dimension of less
+// than 2^32 work-items (2^24 workgroups of 256), so rows past 2^22 continue in y.
+inline dim3 row_grid(int64_t rows) {
+  constexpr int64_t X = 1 << 22;
+  return rows <= X ? dim3((unsigned)rows) : dim3((unsigned)X, (unsigned)((rows + X - 1) / X));
+}
+// The row of this workgroup; the last y holds some past the end.
+__device__ __forceinline__ int64_t grid_row() {
+  return (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));

@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256) quant_rows_vec(const uint16_t* __restrict
                                                       float* __restrict__ scales,
                                                       int64_t m_pad) {
   const int lane = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;  // in the row
-  const int64_t row = WPR == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : (int64_t)blockIdx.x;
+  const int64_t row = WPR == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : grid_row();
   if (row >= m_pad) return;
   if (row >= m) {
     if (lane < 64) pad_row(codes, scales, row, k, lane);
@@ -154,11 +154,11 @@ hipError_t launch_quant_rows(const uint16_t* x, int64_t m, int64_t k, int64_t ld
                        ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
                        ((reinterpret_cast<uintptr_t>(codes) & 7) == 0);
   const int64_t nvec = k / 8;
-  if (aligned && nvec <= 64 * 32 && m_pad < (int64_t(1) << 31)) {  // one workgroup per shared row
+  if (aligned && nvec <= 64 * 32) {
     // Four waves share a row when rows are few, and always above 4096 columns,
     // where one wave's registers for the whole row leave too few waves in flight.
     if (nvec > 64 && (m_pad <= QUANT_SHARED_ROWS || nvec > 512)) {
-      const dim3 rows((unsigned)m_pad);
+      const dim3 rows = row_grid(m_pad);
       if (nvec <= 256) quant_rows_vec<1, 4><<<rows, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
       else if (nvec <= 512) quant_rows_vec<2, 4><<<rows, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);
       else if (nvec <= 1024) quant_rows_vec<4, 4><<<rows, block, 0, s>>>(x, m, k, ldx, codes, scales, m_pad);

@@ -239,7 +239,8 @@ __global__ void __launch_bounds__(256) restore_rows(const uint8_t* __restrict__ 
                                                     const float* __restrict__ sw, int64_t n,
                                                     int64_t k, int64_t ldw,
                                                     uint16_t* __restrict__ out) {
-  const int64_t row = blockIdx.x;
+  const int64_t row = grid_row();
+  if (row >= n) return;
   const float s = sw[row];
   const v4i* src = reinterpret_cast<const v4i*>(w + row * ldw);
   v4i* dst = reinterpret_cast<v4i*>(out + row * k);
@@ -260,7 +261,7 @@ __global__ void __launch_bounds__(256) restore_rows(const uint8_t* __restrict__ 
 
 hipError_t launch_restore_rows(const uint8_t* w, const float* sw, int64_t n, int64_t k, int64_t ldw,
                                uint16_t* out, hipStream_t s) {
-  restore_rows<<<dim3((unsigned)n), dim3(256), 0, s>>>(w, sw, n, k, ldw, out);
+  restore_rows<<<row_grid(n), dim3(256), 0, s>>>(w, sw, n, k, ldw, out);
   return hipGetLastError();
 }
 

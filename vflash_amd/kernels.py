@@ -523,7 +523,7 @@ def weight_only_linear(value, weight, scale, bias=None):
     matrix = value.reshape(-1, k)
     rows = matrix.shape[0]
     ldx, ldw = matrix.stride(0) if rows > 1 else k, weight.stride(0) if n > 1 else k
-    if (k % 16 or n % 8 or rows < 1 or matrix.stride(1) != 1 or ldx < k or ldx % 8 or ldx >= 1 << 22
+    if (k % 16 or n % 8 or n >= 1 << 29 or rows < 1 or matrix.stride(1) != 1 or ldx < k or ldx % 8 or ldx >= 1 << 22
             or weight.stride(1) != 1 or ldw < k or ldw % 16 or ldw >= 1 << 23
             or not scale.is_contiguous() or (bias is not None and not bias.is_contiguous())):
         return None
