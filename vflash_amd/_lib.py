@@ -2,12 +2,15 @@
 
 The library is loaded lazily on first use.  There is no fallback: a missing
 library or a device other than gfx950 raises, so no caller can silently run
-another arithmetic.
+another arithmetic.  The one exception is the weight-only linear, whose
+definition is a torch expression: without the library it runs as that, with a
+warning (``available``).
 """
 
 from __future__ import annotations
 
 import ctypes
+import warnings
 from functools import cache
 from pathlib import Path
 
@@ -121,6 +124,18 @@ def library() -> ctypes.CDLL:
     if lib.vflash_abi_version() != ABI_VERSION:
         raise RuntimeError("libvflash_amd.so has an unexpected ABI version")
     return lib
+
+
+@cache
+def available() -> bool:
+    """Whether the library loads; a warning, once, where it does not.  For calls that
+    are defined without it."""
+    try:
+        library()
+    except (RuntimeError, OSError) as e:
+        warnings.warn(f"{e}; the weight-only linear runs as a torch expression", RuntimeWarning, stacklevel=2)
+        return False
+    return True
 
 
 @cache

@@ -512,11 +512,11 @@ def weight_only_linear(value, weight, scale, bias=None):
     """``F.linear(value, (weight.float() * scale).to(bfloat16), bias)`` as one GEMM that
     restores the weight on the fly, or None where a call is outside the kernel's forms
     (and the caller takes the torch expression): BF16 rows on the current gfx950 device,
-    K % 16 == 0, N % 8 == 0, 16-byte aligned operands with unit column stride, and
-    nothing that records the call (``_eager_inference``)."""
+    K % 16 == 0, N % 8 == 0, 16-byte aligned operands with unit column stride,
+    nothing that records the call (``_eager_inference``), and a library that loads."""
     device = value.device
     if (value.dtype != torch.bfloat16 or not _lib.is_gfx950(device)
-            or not _eager_inference(value, weight, scale, bias)
+            or not _eager_inference(value, weight, scale, bias) or not _lib.available()
             or device.index != torch.cuda.current_device()):
         return None
     n, k = weight.shape
