@@ -2,10 +2,13 @@
 the device and launch checks are answered as a gfx950 device would, and the calls
 must not get as far as a launch."""
 
+import sys
+
 import pytest
 import torch
 
-from vflash_amd import _lib, kernels
+import vflash_amd
+from vflash_amd import _lib, build, fused, kernels
 from vflash_amd.fp8_linear import RowFP8Execution
 from vflash_amd.prepare import quantize_weight_rows
 
@@ -46,3 +49,43 @@ def test_weight_only_without_the_library(monkeypatch, tmp_path, gfx950, fresh):
         assert torch.equal(RowFP8Execution().linear(x, w, s, b), want)
     with pytest.raises(RuntimeError, match="not built"):
         RowFP8Execution("w8a8", activation_quantizer="hip").linear(x, w, s, b)
+
+
+@pytest.fixture
+def no_host(monkeypatch, fresh):
+    """_host.so does not import, as under another Python or torch."""
+    monkeypatch.setitem(sys.modules, "vflash_amd._host", None)
+    monkeypatch.delattr(vflash_amd, "_host", raising=False)
+
+
+def test_w8a8_without_the_host_module(monkeypatch, gfx950, no_host):
+    x, w, s, b = operands()
+    down, up = torch.zeros((8, 32), dtype=torch.bfloat16), torch.zeros((16, 8), dtype=torch.bfloat16)
+    launched = []
+    monkeypatch.setattr(kernels, "call", lambda name, *args: launched.append(name))
+    monkeypatch.setattr(RowFP8Execution, "native", lambda self, value: True)
+    ex = RowFP8Execution("w8a8", activation_quantizer="hip")
+    with pytest.warns(RuntimeWarning, match="native host path is off"):
+        assert ex.linear(x, w, s, b).shape == (5, 16)
+    assert fused.fp8_linear_lora(ex, x, w, s, b, down, up).shape == (5, 16)
+    assert launched == ["vflash_quantize_rows_e4m3", "vflash_fp8_linear", "vflash_quantize_rows_lora_e4m3",
+                        "vflash_fp8_linear_lora"]
+    assert ex.calls == {"weight_only": 0, "w8a8": 2}
+
+
+@pytest.mark.parametrize("absent", ["torch", "torch headers", "Python headers"])
+def test_build_without_what_only_the_host_module_needs(monkeypatch, tmp_path, capsys, absent):
+    stale = tmp_path / "_host.so"
+    stale.write_bytes(b"of another build")
+    monkeypatch.setattr(build, "HOST_MODULE", stale)
+    monkeypatch.setattr(build.subprocess, "run", lambda *a, **k: pytest.fail("nothing to compile"))
+    if absent == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    elif absent == "torch headers":
+        from torch.utils import cpp_extension
+
+        monkeypatch.setattr(cpp_extension, "include_paths", lambda *a, **k: [str(tmp_path)])
+    else:
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build.build_host() is None
+    assert "not built" in capsys.readouterr().err and not stale.exists()

@@ -140,14 +140,19 @@ def available() -> bool:
 
 @cache
 def host():
-    """The native host path (csrc/host.cpp), built next to the library."""
-    library()
+    """The native host path (csrc/host.cpp, _host.so next to the library), or None where
+    it is not built for this Python and torch: the wrappers of ``kernels`` then make the
+    same launches, with more host time per call.  A warning, once, says so.  A library
+    that does not load also gives None, and the wrappers report it."""
     try:
+        library()
         from vflash_amd import _host
     except ImportError as e:
-        raise RuntimeError(
-            "vflash_amd/_host.so is not built for this Python and torch; run `python -m vflash_amd.build`"
-        ) from e
+        warnings.warn(f"the native host path is off ({e}); `python -m vflash_amd.build` builds it for this "
+                      "Python and torch", RuntimeWarning, stacklevel=2)
+        return None
+    except (RuntimeError, OSError):
+        return None
     return _host
 
 

@@ -223,14 +223,28 @@ def _compile(source: Path) -> Path:
     return obj
 
 
-def build_host() -> Path:
+def build_host() -> Path | None:
     """Compile csrc/host.cpp, the native host path (a CPython module on torch's C++
-    API), against the built C-ABI library that sits beside it."""
-    import torch
-    from torch.utils import cpp_extension
+    API), against the built C-ABI library that sits beside it.  None, and no module
+    left from another build, where torch or the C++ headers of torch or Python are
+    absent: the library serves every call without it."""
+    python = sysconfig.get_paths()["include"]
+    try:
+        import torch
+        from torch.utils import cpp_extension
 
+        includes = [*cpp_extension.include_paths(), python]
+    except (ImportError, OSError) as e:
+        includes, missing = [], str(e)
+    else:
+        missing = "".join(f" {h}" for h in ("torch/csrc/autograd/python_variable.h", "Python.h")
+                          if not any((Path(p) / h).exists() for p in includes))
+    if missing:
+        HOST_MODULE.unlink(missing_ok=True)
+        print(f"{HOST_MODULE.name}, the native host path, is not built: missing {missing.strip()}", file=sys.stderr)
+        return None
     source, obj, tmp = CSRC / "host.cpp", OBJECTS / "host.o", HOST_MODULE.with_suffix(".so.tmp")
-    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    includes.append("/opt/rocm/include")
     defines = ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
     libraries = [f"-L{p}" for p in cpp_extension.library_paths()]

@@ -444,7 +444,9 @@ def fp8_linear_lora(
     """
     if strength != 0.0 and execution.observer is None and execution.native(value):
         # The whole call in native code; None sends any other layout on from here.
-        out = _lib.host().w8a8_linear_lora(value, weight, scale, bias, lora_a, lora_b, scaling, strength)
+        host = _lib.host()
+        out = (host.w8a8_linear_lora(value, weight, scale, bias, lora_a, lora_b, scaling, strength)
+               if host is not None else None)
         if out is not None:
             execution.calls["w8a8"] += 1
             return out
