@@ -30,7 +30,7 @@ extern "C" {
 /* Bytes of the static device scratch of vflash_fp8_linear_swiglu_quantize_noalloc. */
 #define VFLASH_NOALLOC_SCRATCH_BYTES (16 << 20)
 
-/* Version of this interface; bumped when a signature changes. */
+/* Version of this interface; bumped when a signature changes (an added entry point changes none). */
 int vflash_abi_version(void);
 
 /* Static string for a status code. */

@@ -1,7 +1,8 @@
-"""What still works when a built part of the package is absent, checked on the CPU:
+"""What happens when a built part of the package is absent or older, checked on the CPU:
 the device and launch checks are answered as a gfx950 device would, and the calls
 must not get as far as a launch."""
 
+import subprocess
 import sys
 
 import pytest
@@ -89,3 +90,20 @@ def test_build_without_what_only_the_host_module_needs(monkeypatch, tmp_path, ca
         monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
     assert build.build_host() is None
     assert "not built" in capsys.readouterr().err and not stale.exists()
+
+
+# An older library: one whose argument lists differ, one of the same version that
+# lacks entries added since, and a library of something else.
+@pytest.mark.parametrize("source,message", [
+    ("int vflash_abi_version(void) { return 3; }", "unexpected ABI version"),
+    ("int vflash_abi_version(void) { return 4; } int vflash_status_string; int vflash_quantize_rows_e4m3;",
+     "older than this package"),
+    ("int other;", "unexpected ABI version"),
+])
+def test_older_library_is_named(monkeypatch, tmp_path, fresh, source, message):
+    (tmp_path / "old.c").write_text(source)
+    old = tmp_path / "libvflash_amd.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", str(old)], check=True)
+    monkeypatch.setattr(_lib, "LIBRARY", old)
+    with pytest.raises(RuntimeError, match=message):
+        _lib.library()

@@ -117,12 +117,19 @@ def library() -> ctypes.CDLL:
             f"{LIBRARY.name} is not built; run `python -m vflash_amd.build` (hipcc, gfx950)"
         )
     lib = ctypes.CDLL(str(LIBRARY))
+    # The version first: it names a library whose argument lists differ.  Entries added
+    # since keep the version, so one that lacks them is found by name.
+    version = getattr(lib, "vflash_abi_version", None)
+    if version is None or version() != ABI_VERSION:
+        raise RuntimeError(f"{LIBRARY.name} has an unexpected ABI version; run `python -m vflash_amd.build`")
     for name, (args, restype) in SIGNATURES.items():
-        fn = getattr(lib, name)
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise RuntimeError(
+                f"{LIBRARY.name} is older than this package (it has no {name}); run `python -m vflash_amd.build`"
+            )
         fn.argtypes = args
         fn.restype = restype
-    if lib.vflash_abi_version() != ABI_VERSION:
-        raise RuntimeError("libvflash_amd.so has an unexpected ABI version")
     return lib
 
 
