@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from tests.conftest import golden
-from vflash_amd import fused, kernels
+from vflash_amd import _lib, fused, kernels
 from vflash_amd.fp8_linear import RowFP8Execution, RowFP8Linear, _quantize_activation_torch
 from vflash_amd.nvfp4_linear import NVFP4Execution, NVFP4Weight
 
@@ -47,6 +47,18 @@ def test_weight_only_output_is_bitwise_the_restored_weight_linear(fp8_matrix, le
     assert got.dtype == dtype and got.shape == (*lead, OUT)
     assert torch.equal(got, want)
     assert ex.calls == {"weight_only": 1, "w8a8": 0}
+
+
+def test_weight_only_compiles_whole_without_a_device_query(monkeypatch):
+    # One graph of the torch expression: nothing in front of it that a compiler
+    # would have to trace through, such as a cached query of the device.
+    monkeypatch.setattr(_lib, "is_gfx950", lambda device: pytest.fail("device query while compiling"))
+    gen = torch.Generator().manual_seed(0)
+    codes = torch.arange(256).reshape(16, 16).to(torch.float8_e4m3fn)
+    scales, value = torch.rand((16, 1), generator=gen), torch.randn((3, 16), generator=gen).to(torch.bfloat16)
+    compiled = torch.compile(lambda v: RowFP8Execution().linear(v, codes, scales), backend="eager", fullgraph=True)
+    with torch.no_grad():
+        assert torch.equal(compiled(value), restored_linear(value, codes, scales, None))
 
 
 def test_weight_only_matches_the_committed_vector():

@@ -106,3 +106,13 @@ def test_infinite_scale_and_k_tail(dev):
     out = RowFP8Execution().linear(x, codes, scale)
     assert bool(torch.isinf(out[:, 3]).all()) and bool((out[:, 3] > 0).all())
     assert bool(torch.isfinite(out[:, [i for i in range(24) if i != 3]]).all())
+
+
+@pytest.mark.parametrize("backend", ["eager", "aot_eager"])
+def test_compiled_calls_are_one_graph_of_the_expression(dev, backend):
+    x, codes, scale, bias = operands(dev, 24, 80, 40)
+    ex = RowFP8Execution()
+    want = torch.nn.functional.linear(x, (codes.float() * scale).to(torch.bfloat16), bias)
+    with torch.no_grad():
+        assert torch.equal(torch.compile(lambda v: ex.linear(v, codes, scale, bias), backend=backend,
+                                         fullgraph=True)(x), want)

@@ -52,6 +52,16 @@ def test_weight_only_without_the_library(monkeypatch, tmp_path, gfx950, fresh):
         RowFP8Execution("w8a8", activation_quantizer="hip").linear(x, w, s, b)
 
 
+def test_weight_only_on_a_torch_that_does_not_name_its_modes(monkeypatch, gfx950):
+    monkeypatch.delattr(torch._C, "_len_torch_dispatch_stack")
+    monkeypatch.setattr(kernels, "_modes_active", kernels._mode_probe())
+    monkeypatch.setattr(kernels, "call", lambda *args: pytest.fail("launched"))
+    x, w, s, b = operands()
+    want = torch.nn.functional.linear(x, (w.float() * s).to(torch.bfloat16), b)
+    with torch.no_grad():
+        assert torch.equal(RowFP8Execution().linear(x, w, s, b), want)
+
+
 @pytest.fixture
 def no_host(monkeypatch, fresh):
     """_host.so does not import, as under another Python or torch."""

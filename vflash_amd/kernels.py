@@ -488,18 +488,34 @@ def _plain(*tensors) -> bool:
     )
 
 
+def _mode_probe():
+    """A function that says whether a dispatch or function mode, a functorch transform
+    or a forward-mode level is active, or None on a torch that does not answer (the
+    names are not public)."""
+    forward_ad = torch.autograd.forward_ad
+    try:
+        dispatch_modes, function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+        transform, _ = torch._C._functorch.peek_interpreter_stack, forward_ad._current_level
+    except AttributeError:
+        return None
+    return lambda: (dispatch_modes() > 0 or function_modes() > 0 or transform() is not None
+                    or forward_ad._current_level >= 0)
+
+
+_modes_active = _mode_probe()
+
+
 def _eager_inference(*tensors) -> bool:
     """True where a call is plain eager arithmetic that nothing records: no gradient
-    or forward-mode tangent to carry, no autocast, mode, tracer or transform active."""
+    or forward-mode tangent to carry, no autocast, mode, tracer or transform active
+    (none that is known to be inactive counts as active)."""
     return not (
-        (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))
-        or torch.is_autocast_enabled("cuda")
+        torch.compiler.is_compiling()
         or torch.jit.is_tracing()
-        or torch.compiler.is_compiling()
-        or torch._C._len_torch_dispatch_stack()
-        or torch._C._len_torch_function_stack()
-        or torch._C._functorch.peek_interpreter_stack() is not None
-        or torch.autograd.forward_ad._current_level >= 0
+        or (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))
+        or torch.is_autocast_enabled("cuda")
+        or _modes_active is None
+        or _modes_active()
     ) and _plain(*tensors)
 
 
@@ -515,8 +531,10 @@ def weight_only_linear(value, weight, scale, bias=None):
     K % 16 == 0, N % 8 == 0, 16-byte aligned operands with unit column stride,
     nothing that records the call (``_eager_inference``), and a library that loads."""
     device = value.device
-    if (value.dtype != torch.bfloat16 or not _lib.is_gfx950(device)
-            or not _eager_inference(value, weight, scale, bias) or not _lib.available()
+    # What records the call is asked first: a compiler then sees the torch expression
+    # alone, and no device query.
+    if (not _eager_inference(value, weight, scale, bias) or value.dtype != torch.bfloat16
+            or not _lib.is_gfx950(device) or not _lib.available()
             or device.index != torch.cuda.current_device()):
         return None
     n, k = weight.shape
