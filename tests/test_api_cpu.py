@@ -7,6 +7,9 @@ it on small tensors; no GPU is involved.  The fixture data (E4M3 codes
 tests/test_fp8_linear.py:13-16, so the expected values there carry over.
 """
 
+from contextlib import nullcontext
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -373,3 +376,13 @@ def test_low_rank_residual_refusals():
                           torch.zeros((inner, 136), dtype=torch.bfloat16), 1.0)
     with pytest.raises(ValueError, match="ranks up to 128"):
         stack_adapters([ok, ok, big], k, 3 * inner)
+
+
+def test_adapter_linear_takes_any_object_with_the_attributes_of_an_execution():
+    execution = SimpleNamespace(mode="w8a8", activation_quantizer="hip", measure=lambda name: nullcontext(),
+                                observer=None, calls={"weight_only": 0, "w8a8": 0})
+    w, s = torch.zeros((16, 16), dtype=torch.float8_e4m3fn), torch.ones((16, 1))
+    adapter = torch.zeros((8, 16), dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="gfx950"):
+        fused.fp8_linear_lora(execution, torch.zeros((2, 16), dtype=torch.bfloat16), w, s, None, adapter,
+                              adapter.T.contiguous())

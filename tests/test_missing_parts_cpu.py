@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import vflash_amd
-from vflash_amd import _lib, build, fused, kernels
+from vflash_amd import _lib, build, fp8_linear, fused, kernels
 from vflash_amd.fp8_linear import RowFP8Execution
 from vflash_amd.prepare import quantize_weight_rows
 
@@ -74,7 +74,8 @@ def test_w8a8_without_the_host_module(monkeypatch, gfx950, no_host):
     down, up = torch.zeros((8, 32), dtype=torch.bfloat16), torch.zeros((16, 8), dtype=torch.bfloat16)
     launched = []
     monkeypatch.setattr(kernels, "call", lambda name, *args: launched.append(name))
-    monkeypatch.setattr(RowFP8Execution, "native", lambda self, value: True)
+    for module in (fp8_linear, fused):
+        monkeypatch.setattr(module, "takes_native_path", lambda execution, value: True)
     ex = RowFP8Execution("w8a8", activation_quantizer="hip")
     with pytest.warns(RuntimeWarning, match="native host path is off"):
         assert ex.linear(x, w, s, b).shape == (5, 16)

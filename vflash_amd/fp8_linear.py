@@ -65,6 +65,19 @@ def _unmeasured(_name: str) -> AbstractContextManager[Any]:
     return nullcontext()
 
 
+def takes_native_path(execution, value) -> bool:
+    """Whether a call may run through the native host path: W8A8 with the HIP
+    quantizer, no scope to open between its kernels, a tensor on a GPU.  Any object
+    with the attributes of a ``RowFP8Execution`` can be asked."""
+    return (
+        execution.mode == "w8a8"
+        and execution.activation_quantizer != "torch"
+        and execution.measure is _unmeasured
+        and isinstance(value, torch.Tensor)
+        and value.is_cuda
+    )
+
+
 def w8a8_supported(value: torch.Tensor) -> bool:
     return value.dtype == torch.bfloat16 and _lib.is_gfx950(value.device)
 
@@ -104,21 +117,10 @@ class RowFP8Execution:
             raise ValueError("unknown FP8 execution mode")
         self.mode = mode
 
-    def native(self, value) -> bool:
-        """Whether a call may run through the native host path: W8A8 with the HIP
-        quantizer, no scope to open between its kernels, a tensor on a GPU."""
-        return (
-            self.mode == "w8a8"
-            and self.activation_quantizer != "torch"
-            and self.measure is _unmeasured
-            and isinstance(value, torch.Tensor)
-            and value.is_cuda
-        )
-
     def linear(self, value, weight, scale, bias=None):
         if self.observer is not None and sum(self.calls.values()) % 200 == 0:
             self.observer()
-        if self.native(value):
+        if takes_native_path(self, value):
             # The whole call in native code; None sends any other layout on from here.
             host = _lib.host()
             output = host.w8a8_linear(value, weight, scale, bias) if host is not None else None

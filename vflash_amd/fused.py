@@ -35,7 +35,7 @@ from dataclasses import dataclass
 import torch
 
 from vflash_amd import _lib, kernels
-from vflash_amd.fp8_linear import RowFP8Execution, _quantize_activation_torch, w8a8_supported
+from vflash_amd.fp8_linear import RowFP8Execution, _quantize_activation_torch, takes_native_path, w8a8_supported
 from vflash_amd.producers import QuantizedRows
 
 
@@ -442,7 +442,7 @@ def fp8_linear_lora(
     ``result + bf16(bf16(bf16(x A^T) B^T) [* scaling] [* strength])``;
     strength 0 skips the adapter (h3_reference_lora.py:75-78).
     """
-    if strength != 0.0 and execution.observer is None and execution.native(value):
+    if strength != 0.0 and execution.observer is None and takes_native_path(execution, value):
         # The whole call in native code; None sends any other layout on from here.
         host = _lib.host()
         out = (host.w8a8_linear_lora(value, weight, scale, bias, lora_a, lora_b, scaling, strength)
