@@ -150,14 +150,18 @@ int vflash_fp8_linear_swiglu_lora(const void* a, const float* sa, int64_t lda, c
 int64_t vflash_swiglu_parts(int64_t n);
 
 /*
- * The tiling vflash_fp8_linear and the other E4M3 GEMM entries use for an
+ * The tiling that vflash_fp8_linear and the other E4M3 GEMM entries choose for an
  * m x n output on a device with `compute_units` CUs (a host-side query; no
  * device work).  0: 256x256, 1: 256x192, 2: 256x128, 3: 128x192, 4: 128x128
  * (two workgroups per CU), 5: 128x128 (one per CU, grids of one round),
- * 6: 128x64, 7: 64x64.  The SwiGLU entries use 256x256 (64x256 in a nearly
- * empty last round).  The plain and gate-residual entries may run 256x256 tiles with
- * a last round of smaller ones where this answers 256x256 or 256x192.  No tiling
- * changes a result bit; this exists so that tests can aim shapes at each one.
+ * 6: 128x64, 7: 64x64.  It is the choice among tilings, and not always the kernel
+ * that runs:
+ *   - outputs of so few rows that ceil(m / 64) * ceil(n / 32) workgroups, of 64 rows
+ *     x 32 columns, get a CU each take a kernel of their own, whatever this answers;
+ *   - the plain and gate-residual entries may run 256x256 tiles with a last round of
+ *     smaller ones where this answers 256x256 or 256x192;
+ *   - the SwiGLU entries use 256x256 (64x256 in a nearly empty last round).
+ * Neither the tiling nor these forms change a result bit.
  * branch_cols > 0 (a multiple of 32): the choice of a LoRA entry with adapter
  * branches that wide: the best of the tilings whose wave width (half the tile width)
  * divides branch_cols (a launch may still run 256x192, whose epilogue splits a wave).

@@ -8,6 +8,7 @@ test sees the stand-in.
 """
 
 import json
+import re
 import subprocess
 import sys
 from pathlib import Path
@@ -65,19 +66,36 @@ lib = ctypes.CDLL(sys.argv[2])
 hip.launched.restype = ctypes.c_char_p
 results = []
 for name, args in json.load(sys.stdin):
-    at = lambda v: ctypes.c_void_p(int(v[1:])) if v[0] == "@" else ctypes.c_float(float(v))
+    def argument(v):
+        if v is None or isinstance(v, int):
+            return v if v is None else ctypes.c_int64(v)
+        if isinstance(v, list):
+            return (ctypes.c_float * len(v))(*v)
+        return ctypes.c_void_p(int(v[1:])) if isinstance(v, str) else ctypes.c_float(v)
     hip.forget()
-    status = getattr(lib, name)(*[at(a) if isinstance(a, str) else None if a is None else ctypes.c_int64(a)
-                                  for a in args])
+    status = getattr(lib, name)(*map(argument, args))
     results.append([status, hip.launched().decode().split("\n")[:-1]])
 json.dump(results, sys.stdout)
 """
 
 
+def kernel_name(mangled):
+    """``fp8_gemm_pipe<0,64,64,4,0,1>`` of a mangled kernel of the library."""
+    head = re.match(r"_ZN3vfa(\d+)", mangled)
+    start, length = head.end(), int(head.group(1))
+    name, rest = mangled[start : start + length], mangled[start + length :]
+    arguments = re.match(r"I((?:L[ib]n?\d+E)+)E", rest)
+    if arguments is None:
+        return name
+    values = [v.replace("n", "-") for v in re.findall(r"L[ib](n?\d+)E", arguments.group(1))]
+    return f"{name}<{','.join(values)}>"
+
+
 def launches(tmp_path, calls):
-    """Run C-ABI calls, ``(entry, arguments)`` with integers as int64, ``"@address"``
-    as a pointer, any other string as a float and None as NULL.  Returns for each
-    its status and its launches ``(kernel, (x, y, z), threads)``."""
+    """Run C-ABI calls, ``(entry, arguments)`` with integers as int64, floats as
+    float, ``"@address"`` as a pointer, lists as arrays of float and None as NULL.
+    Returns for each its status and its launches ``(kernel, (x, y, z), threads)``, the kernel as
+    ``kernel_name`` gives it."""
     stand_in = tmp_path / "hip_stand_in.so"
     source = tmp_path / "hip_stand_in.cpp"
     if not stand_in.exists():
@@ -89,5 +107,5 @@ def launches(tmp_path, calls):
     out = []
     for status, lines in json.loads(done.stdout):
         fields = [line.split() for line in lines]
-        out.append((status, [(f[0], tuple(map(int, f[1:4])), int(f[4])) for f in fields]))
+        out.append((status, [(kernel_name(f[0]), tuple(map(int, f[1:4])), int(f[4])) for f in fields]))
     return out

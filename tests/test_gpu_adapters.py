@@ -137,7 +137,9 @@ def test_qkv_branches_on_the_kernels_operands(dev, m, hidden, inner, ranks, scal
     planes = qkv_linear(ex, xd, w, sc, bias, planes=True, residuals=stacked)
     for got, ref in zip(planes, (q, k, v)):
         assert got.is_contiguous() and torch.equal(got, ref)
-    # The branch width decides the tiling: every wave's columns lie in one branch.
+    # The branch width decides the answer of the query: a tiling whose waves lie in one
+    # branch.  (These shapes run the few-row kernel or such a tiling; 256x192, which may
+    # split a wave, is in test_gpu_lora_tiles.py.)
     tiling = kernels.gemm_tiling(m, 3 * inner, branch_cols=inner)
     wave_cols = int(tiling.split("x")[1].split()[0]) // 2
     assert inner % wave_cols == 0
@@ -233,7 +235,8 @@ def gate_case(m, k, n, rank, scaling, seed, dev, token_gate=False):
 @pytest.mark.parametrize(
     "m,k,n,rank,scaling,token_gate",
     [
-        (300, 512, 640, 16, 0.0625, False),    # 64x64
+        (300, 512, 640, 16, 0.0625, False),    # few-row kernel
+        (300, 512, 2064, 16, 0.0625, False),   # 64x64
         (300, 512, 4112, 5, 1.0, True),        # 128x64
         (2100, 384, 3712, 40, 0.5, False),     # 128x128, two per CU
         (1024, 1536, 6144, 32, 1.375, True),   # 128x192

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 # On 256 CUs 2000 rows (9000 at 48 columns) are tiled; 1 and 17 rows take 32-row
 # workgroups at every width, 40 and 64 rows 32-row ones at 48 and 1008 columns and
-# 64-row ones at 5136.  Widths end inside a 32-column block; K 16 and 144 end
+# 64-row ones at 5136.  300 rows are ten 32-row workgroups high at 48 columns and five
+# 64-row ones at 1008 (128x64 tiles at 5136).  Widths end inside a 32-column block; K 16 and 144 end
 # inside a stage, 1280 runs past the ring.
 @pytest.mark.parametrize("k", [16, 144, 1280])
 @pytest.mark.parametrize("n", [48, 1008, 5136])
@@ -40,6 +41,6 @@ def test_few_rows_match_the_tiled_kernel(dev, k, n):
         yield kernels.fp8_gemm_gate_residual(c, s, w, sw, m, gt, r, bias, lora=lora)
 
     expected = list(calls(whole))
-    for m in (1, 17, 40, 64):
+    for m in (1, 17, 40, 64, 300):
         for i, got in enumerate(calls(m)):
             assert torch.equal(got, expected[i][:m]), (m, i)

@@ -376,11 +376,12 @@ def test_lora_linear_audio_projection_shapes(dev, m, r, scaling, strength):
 
 
 # Tilings with at most eight 32x32 blocks per wave compute the adapter products
-# ahead of the K loop (64x64: 300 x 640, 128x64: 300 x 4112, 128x128:
-# 2100 x 3712, 128x192: 1024 x 6144, 256x128: 1024 x 7168), the others in the
-# epilogue (256x192: 4096 x 3072, 256x256: 4100 x 3088).
+# ahead of the K loop (64x64: 300 x 2064, 128x64: 300 x 4112, 128x128:
+# 2100 x 3712, 128x192: 1024 x 6144, 256x128: 1024 x 7168), as the few-row kernel
+# does (300 x 640), the others after it (256x192: 4096 x 3072) or in the epilogue
+# (256x256: 4100 x 3088).
 @pytest.mark.parametrize("r", [32, 48, 128])
-@pytest.mark.parametrize("m,n,k", [(300, 640, 512), (300, 4112, 512), (2100, 3712, 384),
+@pytest.mark.parametrize("m,n,k", [(300, 640, 512), (300, 2064, 512), (300, 4112, 512), (2100, 3712, 384),
                                    (1024, 6144, 1536), (1024, 7168, 512), (4096, 3072, 1536),
                                    (4100, 3088, 256)])
 def test_lora_epilogue_under_each_tiling(dev, m, n, k, r):
@@ -493,13 +494,14 @@ def test_ffn_with_gate_index_equals_the_gathered_gate(dev):
     assert torch.equal(got, ref)
 
 
-@pytest.mark.parametrize("m,h,k", [(300, 512, 384), (4096, 5120, 256)])
+@pytest.mark.parametrize("m,h,k", [(300, 512, 384), (300, 2064, 384), (4096, 5120, 256), (4096, 3072, 256)])
 def test_gate_residual_operand_layouts_give_the_same_bits(dev, m, h, k):
     # The epilogue loads a residual and a gate chunk with one 16-byte load each
     # when both are 16-byte aligned and the gate has unit column stride, and
     # element by element otherwise; the output takes 16-byte stores when it is
-    # aligned.  Every layout computes the same bits.  The shapes cover whole
-    # and partial 64x64 tiles and the 256x192 tiling's rows past the tile.
+    # aligned.  Every layout computes the same bits.  The shapes cover
+    # the few-row kernel, whole and partial 64x64 tiles, a last round of 128x128 tiles
+    # and 256x192 tiles.
     g = torch.Generator().manual_seed(61)
     x = torch.randn((m, k), generator=g).to(torch.bfloat16).to(dev)
     cw, sw = quantize_weight_rows(torch.randn((h, k), generator=g) * 0.02)

@@ -22,10 +22,14 @@ def tiling(m, n):
 
 
 # Edge shapes under each tiling: partial row and column tiles, K tails
-# (K % 128 != 0 takes the vector-offset DMA everywhere), one K stage.
+# (K % 128 != 0 takes the vector-offset DMA everywhere), one K stage.  The first four
+# run the few-row kernel, which serves shapes of at most 256 of its workgroups whatever
+# the query answers; test_launched_kernels_cpu.py pins what each entry here launches.
 EDGES = [
     (1, 16, 16, "64x64"), (17, 48, 272, "64x64"), (300, 144, 48, "64x64"),
     (257, 256, 528, "64x64"),
+    (1, 16, 8208, "64x64"), (17, 144, 8208, "64x64"), (65, 256, 4112, "64x64"),
+    (257, 48, 2064, "64x64"), (300, 1296, 2064, "64x64"),
     (257, 144, 4112, "128x64"), (300, 256, 4112, "128x64"),
     (520, 144, 4112, "128x128 one round"), (300, 256, 7184, "128x128 one round"),
     (600, 144, 11008, "128x128"), (2100, 256, 3712, "128x128"),

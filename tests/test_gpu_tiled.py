@@ -6,9 +6,11 @@ The reference runs every linear of a block on row tiles of 1024..65536 rows
 token matrix, on 1024-row tiles plus a 17-row remainder, and on 16384-row tiles,
 and the three results must be identical.  The widths are the configuration
 widths (hidden 5120, merged QKV 15360, FFN 13824, adapter K 1536 / N 6144), so
-the automatic GEMM tiling changes with the tile height: 256x256 on the whole
-matrix and on 16384-row tiles, 128x192 for 1024-row tiles of the 5120- and
-6144-wide projections, and 64x64 for the 17-row remainder.
+the GEMM changes with the tile height: 256x256 tiles on the whole matrix and on
+16384-row tiles (with a last round of 256x128 ones where it is at most half full),
+128x192 for 1024-row tiles of the 5120- and 6144-wide projections, and for the
+17-row remainder the few-row kernel at those widths and 64x64 tiles at 13824 and
+15360.
 """
 
 import pytest

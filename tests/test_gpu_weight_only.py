@@ -20,7 +20,7 @@ def operands(dev, m, k, n, seed=0):
 
 
 def check(out, x, codes, scale, bias):
-    """One bf16 rounding (half a step, 2^-9 relative, of the sum) and a binary32 sum
+    """One bf16 rounding (half a step: 2^-8 relative, eight significant bits) and a binary32 sum
     of K products in any order (K 2^-24 of the sum of magnitudes; 2^-23 leaves room
     for the accumulator's own alignment)."""
     w = (codes.float() * scale).to(torch.bfloat16).double()
@@ -34,9 +34,12 @@ def check(out, x, codes, scale, bias):
 
 # Partial tiles in rows and columns, K tails inside a 64-K stage, each tiling
 # (64x64; 128x64 at 200 x 5128; 128x128 at 600 x 5128; 128x256 at 1000 x 7176)
-# and the restoring pass (1025 rows).
+# and the restoring pass (1025 rows).  K = 1296 is 21 stages, the last one partial:
+# every slot of each ring (six slots below 128x128, else four) is refilled more than
+# twice, and the loop over whole rings ends inside one.
 @pytest.mark.parametrize("m,k,n", [(1, 16, 8), (17, 48, 272), (65, 144, 72), (200, 80, 5128),
-                                   (600, 208, 5128), (1000, 272, 7176), (1025, 112, 136)])
+                                   (600, 208, 5128), (1000, 272, 7176), (1025, 112, 136),
+                                   (17, 1296, 272), (200, 1296, 5128), (600, 1296, 5128), (1000, 1296, 7176)])
 @pytest.mark.parametrize("with_bias", [True, False])
 def test_weight_only_linear(dev, m, k, n, with_bias):
     x, codes, scale, bias = operands(dev, m, k, n, seed=m)

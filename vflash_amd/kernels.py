@@ -466,8 +466,9 @@ def fp8_gemm_lora_branches(codes, act_scale, weight, w_scale, rows, t, t_branch,
 
 
 def gemm_tiling(m: int, n: int, compute_units: int = 256, branch_cols: int = 0) -> str:
-    """Name of the tiling the E4M3 GEMM entries use for an m x n output
-    (``vflash_fp8_gemm_tiling``; a host-side query)."""
+    """Name of the tiling the E4M3 GEMM entries choose for an m x n output
+    (``vflash_fp8_gemm_tiling``, a host-side query, whose declaration says which
+    calls run another form)."""
     index = _lib.library().vflash_fp8_gemm_tiling(m, n, compute_units, branch_cols)
     if index < 0:
         raise ValueError("no tiling for these arguments")
