@@ -13,8 +13,9 @@
 // The input y is the bf16 output of the up projection, so GELU is a function of
 // 16 bits: kGeluTanhTable (generated at build time, activation_tables.h) holds
 // its value for every bf16 pattern, the real function rounded to binary32 and
-// then to bf16.  Each workgroup copies the 128 KB table into LDS once (all
-// of its DMA and the first rows' loads in flight together) and looks every element up with one LDS read; the kernel's work is then HBM-bound.
+// then to bf16.  Each workgroup copies the 128 KB table into LDS once (all of its
+// DMA and the first rows' loads in flight together) and looks every element up
+// with one LDS read; the kernel's work is then HBM-bound.
 //
 // Layout: one workgroup per CU (the table takes 128 KB of the 160 KB LDS), 12
 // waves (three per SIMD), one row per WPR waves at a time with the whole row in

@@ -130,6 +130,10 @@ int tiling_group_m(int tiling, int64_t tile_cols) {
 // 111 and at K = 13824 259 -> 241.  More left than that is slower: 4200 x 5376 x
 // 5376 102 -> 115 (1.40 rounds), 12000 x 5120 x 13824 606 -> 618 (9.91), 5000 x 5120
 // x 5120 112 -> 124 (1.56).
+// Only K % 128 == 0, whose whole tiles run the split ring: any other K takes the
+// two-slot ring in every tile, and no mixed kernel is built or measured on that
+// one.  The adapter epilogues have none either: their tiles of either size would
+// need the adapter products in both halves of the kernel, which was not tried.
 static int mixed_tail(const GemmParams& p, int tiling, int64_t tiles, int64_t cus) {
   const int64_t full = tiles / cus, rem = tiles % cus;
   if (p.k % 128 || rem == 0 || full < 1) return MIXED_NONE;
@@ -143,6 +147,10 @@ static int mixed_tail(const GemmParams& p, int tiling, int64_t tiles, int64_t cu
 // 55.0, 48.6; 1100 179, 155 (two rounds and 48 tiles); 3000 382, 356; at 300 x 2048
 // x 4096 28.8, 15.1.  With more than a round of them: 300 rows 59.3, 91.7; 777
 // rows 127, 140; 1024 131, 149.
+// The limit of eight whole rounds is no measured crossing: past it the share that a
+// split can save only shrinks.  Without the limit, whole and split: 5376 rows 659,
+// 634 (9.2 rounds); 7680 925, 902 (13.1); 14080 1664, 1638 (24.1); 30464 3590, 3554
+// (52.1).  Other K than multiples of 128, and the adapter form: as at mixed_tail.
 static int64_t swiglu_main_tiles(const GemmParams& p, int64_t cus) {
   if (p.k % 128) return -1;
   const int64_t tiles_m = (p.m + 255) / 256, tiles_n = p.half_n / 128, tiles = tiles_m * tiles_n;

@@ -1,6 +1,7 @@
 // A 256x256 grid of the W8A8 E4M3 GEMM whose last round is split into smaller
-// tiles (fp8_gemm_mixed.hip instantiates it per epilogue; fp8_gemm.hip, mixed_tail,
-// chooses it).  Kernel-side only; not part of the C-ABI.
+// tiles (instantiated per epilogue in fp8_gemm_mixed_bias.hip, fp8_gemm_mixed_gate.hip
+// and fp8_gemm_mixed_swiglu.hip; fp8_gemm.hip chooses it, mixed_tail and
+// swiglu_main_tiles).  Kernel-side only; not part of the C-ABI.
 #pragma once
 #include "fp8_gemm_pipe.h"
 

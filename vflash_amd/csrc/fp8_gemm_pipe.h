@@ -243,11 +243,14 @@ __device__ __forceinline__ void pipe_tile(const GemmParams& p, int tm, int tn, u
 
   // Tiles of at most eight 32x32 blocks per wave compute their adapter products
   // before the K loop (up to 128 registers held through it), so the epilogue
-  // does not wait on their loads.  The 256x192 tile, whose registers hold the
-  // main loop, computes them after it from LDS (192 registers that the dead
-  // fragments leave free): 126 us against 148 with a gather per block at 1024 x
-  // 5376 x 21504, rank 128.  The 256x256 tile's 256 do not fit beside the
-  // accumulators and are formed block by block in the epilogue.
+  // does not wait on their loads; they stand ahead of the first stages' DMA and
+  // do not overlap it.  The 256x192 tile, whose registers hold the main loop,
+  // computes them after it from LDS: 126 us against 148 with a gather per block at
+  // 1024 x 5376 x 21504, rank 128.  Its 192 registers of products beside the 192
+  // accumulators spill 132 bytes a lane (split ring; the two-slot form spills
+  // none), and their DMA starts only when the K loop has ended.  The 256x256
+  // tile's 256 do not fit beside the accumulators and are formed block by block
+  // in the epilogue.
   constexpr bool LORA_PRE = epi_lora(EPI) && MB * NB <= 8;
   constexpr bool LORA_POST = epi_lora(EPI) && !LORA_PRE && MB * NB <= 12;
   static_assert(!LORA_POST || (BM + BN) * 256 <= (SPLIT ? (2 * BM + 2 * BN) * 128 : pipe_lds(BM, BN, NS)),

@@ -2,9 +2,10 @@
 // allocations and launches of one call without a round trip through Python for
 // each of them.
 //
-// A 17-row linear keeps the GPU busy for 15 us, while the Python wrappers of its
-// two kernels (argument checks, four allocations, two ctypes calls) took 25 us of
-// host time, and the adapter linear's 36 us against 18.  Each function here takes
+// A 17 x 5120 x 5120 linear keeps the GPU busy for 11 us, while the Python wrappers
+// of its two kernels (argument checks, four allocations, two ctypes calls) take 24 us
+// of host time; here it takes 10.  The adapter linear: 16 us of GPU time at 256 x 1536
+// x 4608, 34 us of host time in the wrappers, 11 here.  Each function here takes
 // the tensors of a call, and either runs the whole of it on the tensor's current
 // stream or returns None without having enqueued anything that the caller sees:
 // every other layout, type, device or error goes on to the Python wrappers, which

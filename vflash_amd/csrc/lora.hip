@@ -37,8 +37,8 @@
 namespace vfa {
 
 constexpr int LD_WAVES = 8;
-constexpr int LD_ROWS = 16;   // rows of x per workgroup
-constexpr int LD_RANKS = 16;  // adapter rows per workgroup
+constexpr int LD_ROWS = 16;   // rows of x per block
+constexpr int LD_RANKS = 16;  // adapter rows per block
 
 template <bool QUANT, int RW, int RK>
 __global__ void __launch_bounds__(64 * LD_WAVES) lora_down_blocks(

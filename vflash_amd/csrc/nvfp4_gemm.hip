@@ -20,8 +20,8 @@
 namespace vfa {
 
 // ---------------------------------------------------------------------------
-// Pipelined W4A8 kernel (tiles of 64x64 to 256x256): packed operands in LDS, dequantization in
-// registers, f16 MFMA.
+// Pipelined W4A8 kernel (tiles of 64x64 to 256x256): packed operands in LDS,
+// dequantization in registers, f16 MFMA.
 //
 // Every E4M3 code and every product e2m1 * e4m3 (at most 6 significant bits,
 // magnitude 2^-10 .. 2688) is exact in binary16, so the contraction runs on

@@ -34,11 +34,11 @@ __device__ __forceinline__ float half_hi(uint32_t w) {
 // One wave per row segment, four rows per workgroup; gridDim.y splits each row
 // into runs of whole 64-element groups (blocks are independent, and few rows
 // would leave the GPU idle otherwise).  Lane l of pass t reads the 8 elements
-// 512 t + 8 l .. +7 of the segment (16 bytes; four passes' loads are in flight; the wave reads 1 KB contiguously), so
-// a 16-element block is a lane pair: the block maximum takes one shuffle, and
-// each lane writes its 4 packed bytes.  The four scales of a 128x4 word (four
-// consecutive blocks) come from lanes 8u, 8u + 2, 8u + 4, 8u + 6 and are
-// written by lane 8u.
+// 512 t + 8 l .. +7 of the segment (16 bytes; the wave reads 1 KB contiguously,
+// four passes' loads in flight), so a 16-element block is a lane pair: the block
+// maximum takes one shuffle, and each lane writes its 4 packed bytes.  The four
+// scales of a 128x4 word (four consecutive blocks) come from lanes 8u, 8u + 2,
+// 8u + 4, 8u + 6 and are written by lane 8u.
 template <bool F16>
 __global__ void __launch_bounds__(256) nvfp4_quant_rows(const uint16_t* __restrict__ x, int64_t m,
                                                         int64_t k, int64_t ldx,
@@ -121,10 +121,10 @@ hipError_t launch_nvfp4_quant(const uint16_t* x, bool f16, int64_t m, int64_t k,
   const dim3 grid((unsigned)((m_pad + 3) / 4), row_segments(m_pad, k));
   if (f16)
     nvfp4_quant_rows<true><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad,
-                                        alpha, out_scale);
+                                                alpha, out_scale);
   else
     nvfp4_quant_rows<false><<<grid, 256, 0, s>>>(x, m, k, ldx, global_sf, codes, ldc, scales, m_pad,
-                                        alpha, out_scale);
+                                                 alpha, out_scale);
   return hipGetLastError();
 }
 

@@ -144,7 +144,10 @@ unsigned row_segments(int64_t rows, int64_t k) {
 // Rows up to which the four waves of a workgroup share one row at any width.
 // Microseconds unshared -> shared: 300 x 5376 9.5 -> 4.8, 2048 x 5120 11.9 -> 9.1,
 // 32760 x 5120 90 -> 79, 32760 x 14336 387 -> 262, 4095 x 13824 50 -> 33; narrow rows
-// of long calls lose: 4095 x 1536 6.8 -> 7.3, 32760 x 1536 27 -> 38, x 3072 54 -> 55.
+// of long calls lose: 4095 x 1536 6.8 -> 7.3, 4096 x 3072 10.1 -> 10.4, 8192 x 2304
+// 13.6 -> 15.6, 32760 x 1536 27 -> 38, x 3072 57 -> 57.  Close to either line the
+// shared form is still ahead: 2064 x 3072 7.8 -> 6.9, 4096 x 4096 12.6 -> 11.7, 32760 x
+// 4096 69 -> 65.
 constexpr int64_t QUANT_SHARED_ROWS = 2048;
 
 hipError_t launch_quant_rows(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
