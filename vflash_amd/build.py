@@ -2,8 +2,8 @@
 
 Usage: ``python -m vflash_amd.build`` (or ``build()`` from Python).  Each
 ``csrc/*.hip`` file compiles to an object in parallel, then one shared library
-is linked next to this file, where :mod:`vflash_amd._lib` loads it, and the native
-host path (``csrc/host.cpp``, ``_host.so``) against it.
+is linked next to this file, where :mod:`vflash_amd._lib` loads it, and, where torch's
+C++ headers are present, the native host path (``csrc/host.cpp``, ``_host.so``) against it.
 """
 
 from __future__ import annotations
